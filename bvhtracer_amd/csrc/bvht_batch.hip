@@ -126,7 +126,8 @@ __global__ void k_batch_bounds(const BatchScene* __restrict__ scenes, const uint
 __global__ __launch_bounds__(kRebuildWG) void k_batch_rebuild(const BatchScene* __restrict__ scenes)
 {
     BatchScene sc = scenes[blockIdx.x];
-    tlas_rebuild_block(sc.bounds, sc.n_obj, sc.nodes_w, sc.list, sc.meta);
+    extern __shared__ float rebuild_lds[];
+    tlas_rebuild_block(sc.bounds, sc.n_obj, sc.nodes_w, sc.list, sc.meta, rebuild_lds);
 }
 
 template <int WG, int LDS_DEPTH, int RPI>
@@ -219,6 +220,7 @@ struct bvht_batch_s {
     std::vector<uint32_t> refit_off;     // level L occupies [refit_off[L], refit_off[L+1])
     uint32_t* d_obj_prefix = nullptr;
     uint32_t total_nodes = 0, total_objs = 0;
+    size_t rebuild_lds = 0;  // dynamic LDS of k_batch_rebuild: the largest scene's list
     uint32_t cap = 0;  // traversal stack bound: max over scenes of (objects - 1) + (BLAS depth - 1)
     // trace tables (bvht_batch_set_rays)
     uint32_t* d_items = nullptr;
@@ -300,6 +302,7 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
         d.list = t->d_list;
         d.meta = t->d_meta;
         d.n_obj = t->n;
+        b->rebuild_lds = std::max(b->rebuild_lds, rebuild_lds_bytes(t->n));
         d.pad = 0;
         obj_prefix[s + 1] = obj_prefix[s] + t->n;
         uint32_t cap = (t->n - 1) + (t->max_blas_depth > 0 ? t->max_blas_depth - 1 : 0);
@@ -444,8 +447,8 @@ int32_t bvht_batch_rebuild(bvht_ctx ctx, bvht_batch b)
     }
     hipLaunchKernelGGL(k_batch_bounds, dim3(nblk(b->total_objs, 64)), dim3(64), 0, ctx->stream, b->d_scenes,
                        b->d_obj_prefix, (uint32_t)b->scenes.size());
-    hipLaunchKernelGGL(k_batch_rebuild, dim3((uint32_t)b->scenes.size()), dim3(kRebuildWG), 0, ctx->stream,
-                       b->d_scenes);
+    hipLaunchKernelGGL(k_batch_rebuild, dim3((uint32_t)b->scenes.size()), dim3(kRebuildWG), b->rebuild_lds,
+                       ctx->stream, b->d_scenes);
     BVHT_HIP(hipGetLastError());
     return BVHT_OK;
 }

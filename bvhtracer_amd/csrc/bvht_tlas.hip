@@ -36,7 +36,8 @@ __global__ void k_object_bounds(const bvht_instance* __restrict__ objs, uint32_t
 __global__ __launch_bounds__(kRebuildWG) void k_tlas_rebuild(const float* __restrict__ bounds, uint32_t n,
                                                              bvht_tnode* nodes, int32_t* list, uint32_t* meta)
 {
-    tlas_rebuild_block(bounds, n, nodes, list, meta);
+    extern __shared__ float rebuild_lds[];
+    tlas_rebuild_block(bounds, n, nodes, list, meta, rebuild_lds);
 }
 
 template <int WG, int LDS_DEPTH, bool STATS, bool PACKED>
@@ -179,8 +180,8 @@ int32_t refresh(bvht_tlas t)
 
 int32_t rebuild(bvht_tlas t, bool read_depth)
 {
-    hipLaunchKernelGGL(k_tlas_rebuild, dim3(1), dim3(kRebuildWG), 0, t->ctx->stream, t->d_bounds, t->n, t->d_nodes,
-                       t->d_list, t->d_meta);
+    hipLaunchKernelGGL(k_tlas_rebuild, dim3(1), dim3(kRebuildWG), rebuild_lds_bytes(t->n), t->ctx->stream,
+                       t->d_bounds, t->n, t->d_nodes, t->d_list, t->d_meta);
     BVHT_HIP(hipGetLastError());
     if (read_depth) {
         uint32_t meta[3];

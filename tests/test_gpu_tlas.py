@@ -107,6 +107,44 @@ def test_tlas_rebuild_at_the_wave_limit_chains_and_ties(ctx, orc, case):
     assert (got["prim"] != B.MISS).sum() > 100
 
 
+@pytest.mark.parametrize("case", ["random66", "random257", "random2047", "random2048", "random2049", "lattice1000",
+                                  "chain120"])
+def test_tlas_rebuild_in_lds_and_beyond(ctx, orc, case):
+    """65 to 2048 objects keep the merge loop's list in LDS, more in global
+    memory.  Entry counts around a multiple of the workgroup's threads and
+    around the limit, a lattice of equal boxes (every find ties, across lanes
+    and waves: first index) and a chain (its depth, tracked instead of walked,
+    sizes the traversal's stack): nodes bit for bit, hits along the objects."""
+    n = int(case.lstrip("abcdefghijklmnopqrstuvwxyz"))
+    if case.startswith("random"):
+        M, Minv = scenes.random_affines(n, 0xB0D5 + n, trans_range=60.0)
+    elif case.startswith("lattice"):
+        k = np.arange(n)
+        M, Minv = translated(np.stack([k % 10, k // 10 % 10, k // 100], 1) * 8.0 - 36.0)
+    else:
+        gaps = 7.0 * 1.1 ** np.arange(n)
+        M, Minv = translated([(x, 0.0, 0.0) for x in np.cumsum(gaps) - gaps.sum() / 2])
+    mesh = scenes.icosphere(4, radius=3.0, seed=7)
+    nodes, used, perm = orc.bvh_build(mesh, False, 2)
+    model = B.Bvh.from_arrays(nodes, used, perm, ctx=ctx)
+    objs = [B.SceneObject(0, M[k].reshape(4, 4), Minv[k]) for k in range(n)]
+    tlas = B.TlasBuilder(ctx=ctx).build_for(objs, [model])
+    tnodes, t_used = oracle_tlas(orc, [(nodes, perm)], objs)
+    g_nodes, g_used = tlas.download()
+    assert g_used == t_used == 2 * n
+    assert g_nodes.tobytes() == tnodes.tobytes()
+    rays = np.zeros(n, B.RAY_DTYPE)
+    rays["o"] = M[:, 12:15] + np.float32([0.0, 0.0, -50.0])
+    rays["o"][::2] += np.float32([-50.0, 0.3, 50.0])
+    rays["d"] = (0.0, 0.0, 1.0)
+    rays["d"][::2] = (1.0, 0.0, 0.0)
+    rays["tmax"] = np.float32(3.4028235e38)
+    ref = orc.tlas_trace(tnodes, oracle_instances(orc, objs), [(nodes, perm)], rays.view(orc.RAY_DTYPE), nthreads=8)
+    got = tlas.intersect(rays)
+    assert_hits_equal(got, ref, f"tlas {case}")
+    assert (got["prim"] != B.MISS).sum() > n // 4
+
+
 def test_tlas_frame_refit_refresh_rebuild_bounce(ctx, orc):
     """Per frame: deform the shared model, refit it, refresh the object
     bounds (set_transform with the same transform), rebuild the TLAS, trace
