@@ -329,7 +329,12 @@ class SceneObject:
 
 
 def _instances(objects):
-    return np.concatenate([o.record() for o in objects]) if objects else np.zeros(0, INSTANCE_DTYPE)
+    r = np.zeros(len(objects), INSTANCE_DTYPE)
+    if objects:
+        r["m"] = np.concatenate([o.m for o in objects]).reshape(-1, 16)
+        r["minv"] = np.concatenate([o.minv for o in objects]).reshape(-1, 16)
+        r["blas"] = [o.model for o in objects]
+    return r
 
 
 class Tlas:
