@@ -250,18 +250,18 @@ __global__ void k_level_scatter(uint32_t nodes_used, uint32_t depth, const uint3
     }
 }
 
-// Leaves with more than kBigLeaf triangles: counted, then listed.  `wide`
-// (when given) is set if some leaf has 64 or more triangles, too many for a
-// packed stack entry.
+// Leaves with more than kBigLeaf triangles: counted, then listed.  `widest`
+// (when given, 0 before) becomes the triangle count of the largest leaf of at
+// least `from` triangles.
 __global__ void k_big_leaves(const bvht_node* __restrict__ nodes, uint32_t nodes_used, uint32_t* __restrict__ counter,
-                             uint32_t* __restrict__ list, uint32_t* __restrict__ wide)
+                             uint32_t* __restrict__ list, uint32_t* __restrict__ widest, uint32_t from)
 {
     uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nodes_used || k == 1)
         return;
     uint32_t c = nodes[k].count;
-    if (wide && c >= 64u)
-        *wide = 1u;
+    if (widest && c >= from && c > __hip_atomic_load(widest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(widest, c);
     if (c <= kBigLeaf)
         return;
     uint32_t slot = atomicAdd(counter, 1u);
@@ -350,6 +350,29 @@ __global__ __launch_bounds__(WG) void k_trace_blas(const float4* __restrict__ no
         uint64_t dt = (uint64_t)wall_clock64() - t0;
         cost[group] = dt > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)dt;
     }
+}
+
+// k_trace_blas for trees with large leaves: G lanes a ray (traverse_group), a
+// stack of kGroupStack entries a ray in LDS.
+constexpr int kGroupStack = 64;
+
+template <int G>
+__global__ __launch_bounds__(256) void k_trace_group(const float4* __restrict__ nodes, const float* __restrict__ tris,
+                                                     const bvht_ray* __restrict__ rays, bvht_hit* __restrict__ hits,
+                                                     uint32_t n, const uint32_t* __restrict__ d_n,
+                                                     uint32_t* __restrict__ spill, uint32_t cap,
+                                                     uint32_t* __restrict__ status)
+{
+    constexpr int kRays = 256 / G;
+    __shared__ uint32_t lds[kGroupStack * kRays];
+    const uint32_t i = blockIdx.x * kRays + threadIdx.x / G;
+    const uint32_t count = d_n ? min(*d_n, n) : n;
+    if (i >= count)
+        return;
+    Stack<kGroupStack, kRays> st{(lds_u32*)(lds + threadIdx.x / G), spill + i, (size_t)n, cap, status};
+    const BlasResult r = traverse_group<G>(nodes, tris, load_ray(rays, i), st);
+    if (threadIdx.x % G == 0)
+        store_hit(hits, i, r.found, r.t, r.u, r.v, r.prim, 0);
 }
 
 typedef void (*trace_blas_fn)(const float4*, const float*, const bvht_ray*, bvht_hit*, uint32_t, const uint32_t*,
@@ -1254,6 +1277,10 @@ int32_t device_to_host_beside(bvht_ctx ctx, void* dst, const void* src, size_t b
     return device_to_host_on(ctx, cs, dst, src, bytes);
 }
 
+// Triangles of a leaf on average (nodes_used counts the dummy: two a leaf).
+static uint32_t mean_leaf(bvht_blas b) { return b->n_tris / std::max(1u, b->nodes_used / 2); }
+constexpr uint32_t kGroupLeaf = 6;  // mean from which leaf_group considers a group of lanes
+
 int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_depth)
 {
     bvht_ctx ctx = b->ctx;
@@ -1264,7 +1291,7 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     uint32_t nb = blocks_for(b->nodes_used, 256);
     hipLaunchKernelGGL(k_parents, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, b->d_parent);
     // scratch: [0] depth, then the per-level counts, then the big-leaf count
-    // and the wide-leaf flag
+    // and the widest leaf
     rc = ensure_scratch(ctx, sizeof(uint32_t) * (2 * (size_t)b->nodes_used + 4));
     if (rc)
         return rc;
@@ -1283,7 +1310,7 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
         return set_error(BVHT_EDEVICE, "BLAS topology: depth %u out of range", depth);
     b->depth = depth;
     uint32_t* hist = d_depth + 1;
-    uint32_t* big = hist + depth;  // big-leaf count, wide-leaf flag
+    uint32_t* big = hist + depth;  // big-leaf count, widest leaf
     rc = fill_u32(ctx, hist, 0, depth + 2);
     if (rc)
         return rc;
@@ -1291,7 +1318,8 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     hipLaunchKernelGGL(k_level_hist, dim3(nb_levels), dim3(256), 0, st, b->nodes_used, depth, b->d_level, hist);
     // big leaves: counted here, listed below; and whether every node fits a
     // packed stack entry
-    hipLaunchKernelGGL(k_big_leaves, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, big, nullptr, big + 1);
+    hipLaunchKernelGGL(k_big_leaves, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, big, nullptr, big + 1,
+                       mean_leaf(b) >= kGroupLeaf ? 1u : 64u);
     BVHT_HIP(hipGetLastError());
     std::vector<uint32_t> h(depth + 2);
     BVHT_HIP(hipMemcpyAsync(h.data(), hist, sizeof(uint32_t) * (depth + 2), hipMemcpyDeviceToHost, st));
@@ -1307,7 +1335,8 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
                        b->d_level_order);
     BVHT_HIP(hipGetLastError());
     uint32_t nbig = h[depth];
-    b->packed_stack = h[depth + 1] == 0 && b->nodes_used <= kPackMask + 1u && b->n_tris <= kPackMask + 1u;
+    b->widest_leaf = h[depth + 1];
+    b->packed_stack = b->widest_leaf < 64 && b->nodes_used <= kPackMask + 1u && b->n_tris <= kPackMask + 1u;
     (void)hipFree(b->d_big_leaves);
     b->d_big_leaves = nullptr;
     b->n_big_leaves = nbig;
@@ -1318,7 +1347,7 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
         if (rc)
             return rc;
         hipLaunchKernelGGL(k_big_leaves, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, big,
-                           b->d_big_leaves, nullptr);
+                           b->d_big_leaves, nullptr, 0u);
         BVHT_HIP(hipGetLastError());
     }
     BVHT_HIP(hipStreamSynchronize(st));
@@ -1459,6 +1488,34 @@ void trace_config(bvht_ctx ctx, uint32_t need, int* wg, int* lds)
     *lds = need <= 8 ? 8 : (need <= 16 ? 16 : 24);
 }
 
+// Lanes a ray for a trace of n rays over a tree with large leaves, 0 for the
+// lane-a-ray kernel.  A lane with a leaf of hundreds of triangles holds its
+// wave for all of them, and the longest such wave is the launch.  Measured (us,
+// a lane a ray / 8 lanes / 16 lanes) on the reference builder's trees of soups
+// and icospheres, named with their triangles (mean and largest leaf):
+//   7,500 camera rays: soup 12,583 (52, 707) 1875 / 181 / 92, sphere 12,000
+//     (443, 681) 1453 / 138 / 74, sphere 500 (19, 32) 52 / 13 / 11;
+//   409,600, uneven leaves: soup 12,583 3092 / 243 / 168, 3,000 (24, 191)
+//     1223 / 125 / 109, 800 (12, 65) 271 / 74 / 74, 300 (6.2, 29) 93 / 37 / 50;
+//     1.92M: soup 12,583 2729 / 426 / 486;
+//   409,600, even leaves: sphere 12,000 1920 / 567 / 717, 2,000 (80, 134)
+//     195 / 151 / 216, 1,000 (38, 70) 101 / 109 / 162, 500 47 / 91 / 146.
+// So 16 lanes for launches that leave the chip idle; else a group where the
+// leaves are uneven, 16 lanes while each lane still has two triangles a leaf
+// and the waves have not filled the chip; and 8 for even leaves from a mean of
+// 64, below which a wave's lanes are busy together as they are.
+static int leaf_group(bvht_blas b, uint32_t n)
+{
+    const uint32_t mean = mean_leaf(b);
+    if (mean < kGroupLeaf)
+        return 0;
+    if (n <= 65536)
+        return 16;
+    if (b->widest_leaf >= 4 * mean)
+        return mean >= 24 && n <= (1u << 20) ? 16 : 8;
+    return mean >= 64 ? 8 : 0;
+}
+
 int32_t launch_trace_blas(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_rays, uint32_t n,
                           const uint32_t* d_n, bvht_hit* d_hits, bvht_stats* d_stats)
 {
@@ -1468,12 +1525,24 @@ int32_t launch_trace_blas(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_rays, 
     uint32_t need = stack_cap(ctx, blas->depth > 0 ? blas->depth - 1 : 0);
     int wg, lds;
     trace_config(ctx, need, &wg, &lds);
+    // (a stack limit below the tree's bound limits the lane-a-ray kernel's stack)
+    const bool capped = ctx->stack_limit && ctx->stack_limit + 1 < blas->depth;
+    const int group = capped || d_stats || ctx->trace_wg > 0 || ctx->tls_on ? 0 : leaf_group(blas, n);
+    if (group)
+        lds = kGroupStack;
     uint32_t* spill = nullptr;
     if (need > (uint32_t)lds) {
         int32_t rc = ensure_spill(ctx, &ctx->spill, &ctx->spill_words, (size_t)(need - lds) * n);
         if (rc)
             return rc;
         spill = ctx->spill;
+    }
+    if (group) {
+        hipLaunchKernelGGL(group == 16 ? k_trace_group<16> : k_trace_group<8>, dim3(blocks_for(n, 256 / group)),
+                           dim3(256), 0, ctx->stream, reinterpret_cast<const float4*>(blas->d_nodes), blas->d_tris,
+                           d_rays, d_hits, n, d_n, spill, need, ctx->d_status);
+        BVHT_HIP(hipGetLastError());
+        return BVHT_OK;
     }
     trace_blas_fn fn = pick_trace_blas(wg, lds, d_stats != nullptr, blas->packed_stack);
     if (!fn)

@@ -118,6 +118,7 @@ struct bvht_blas_s {
     std::vector<uint32_t> level_off;    // level L occupies [level_off[L], level_off[L+1]) of d_level_order
     uint32_t* d_big_leaves = nullptr;   // leaves with more than kBigLeaf triangles (refit a wave each)
     uint32_t n_big_leaves = 0;
+    uint32_t widest_leaf = 0;   // triangles of the largest leaf (0 if below 64 and leaves are small on average)
     bool packed_stack = false;  // every node fits a packed stack entry (see bvht_trace.hpp)
     // shading attributes (bvht_blas_set_attributes)
     float* d_attr_normals = nullptr;

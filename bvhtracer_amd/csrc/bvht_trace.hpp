@@ -223,6 +223,81 @@ __device__ __forceinline__ BlasResult traverse_blas(const float4* __restrict__ n
     return res;
 }
 
+// Bvh::intersect_subtree with G lanes a ray (4, 8 or 16, aligned), for trees
+// with large leaves: every lane of a group holds the same ray and state and
+// takes the same node steps, and a leaf's triangles are tested G at a time.
+// The nearest accepted triangle, the first of equal ones, is the one the
+// sequential loop keeps.  Its t, u and v come from testing it once more at the
+// end (the same arithmetic).  `st` is the group's one stack.
+template <int G, class StackT>
+__device__ __forceinline__ BlasResult traverse_group(const float4* __restrict__ nodes, const float* __restrict__ tris,
+                                                     const DRay& ray, StackT& st)
+{
+    static_assert(G == 4 || G == 8 || G == 16, "groups within a 16-lane row");
+    const uint32_t lane = threadIdx.x & 63u, sub = lane & (G - 1);
+    float closest = ray.t;
+    uint32_t sp = 0, prim = BVHT_MISS;
+    uint32_t lf = __float_as_uint(nodes[0].w);
+    uint32_t cnt = __float_as_uint(nodes[1].w);
+    while (true) {
+        while (cnt == 0) {
+            const float4* c = nodes + 2 * (size_t)lf;
+            const float4 a0 = c[0], a1 = c[1], b0 = c[2], b1 = c[3];
+            float dl, dr;
+            const bool hl = slab(a0, a1, ray, closest, dl);
+            const bool hr = slab(b0, b1, ray, closest, dr);
+            const float kl = hl ? dl : kFltMax, kr = hr ? dr : kFltMax;
+            const bool left_near = kl < kr;
+            if (left_near ? hl : hr) {
+                if (left_near ? hr : hl)
+                    st.push(sp, left_near ? lf + 1 : lf);
+                const uint32_t nlf = __float_as_uint(left_near ? a0.w : b0.w);
+                cnt = __float_as_uint(left_near ? a1.w : b1.w);
+                lf = nlf;
+            } else {
+                cnt = kPopNext;
+            }
+        }
+        if (cnt != kPopNext) {
+            float bt = closest;
+            uint32_t bi = BVHT_MISS;
+            for (uint32_t k = sub; k < cnt; k += G) {
+                float t, u, v;
+                if (tri_test(tris + 9 * (size_t)(lf + k), ray, t, u, v) && t < bt) {
+                    bt = t;
+                    bi = lf + k;
+                }
+            }
+            auto take = [&](uint32_t ot, uint32_t oi) {
+                const float o = __uint_as_float(ot);
+                if (o < bt || (o == bt && oi < bi)) {
+                    bt = o;
+                    bi = oi;
+                }
+            };
+            take(xor_lane<1>(__float_as_uint(bt), lane), xor_lane<1>(bi, lane));
+            take(xor_lane<2>(__float_as_uint(bt), lane), xor_lane<2>(bi, lane));
+            if constexpr (G >= 8)
+                take(xor_lane<4>(__float_as_uint(bt), lane), xor_lane<4>(bi, lane));
+            if constexpr (G >= 16)
+                take(xor_lane<8>(__float_as_uint(bt), lane), xor_lane<8>(bi, lane));
+            if (bi != BVHT_MISS) {
+                closest = bt;
+                prim = bi;
+            }
+        }
+        if (sp == 0)
+            break;
+        const uint32_t e = st.pop(sp);
+        lf = __float_as_uint(nodes[2 * (size_t)e].w);
+        cnt = __float_as_uint(nodes[2 * (size_t)e + 1].w);
+    }
+    BlasResult res{0.0f, 0.0f, 0.0f, prim, false};
+    if (prim != BVHT_MISS && closest < kFltMax)
+        res.found = tri_test(tris + 9 * (size_t)prim, ray, res.t, res.u, res.v);
+    return res;
+}
+
 // Per-BLAS device pointers used by the TLAS kernels.
 struct BlasRef {
     const float4* nodes;

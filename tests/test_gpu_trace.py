@@ -506,3 +506,43 @@ def test_trace_after_refit_sees_the_new_boxes(ctx, orc):
         ref = orc.bvh_trace(ref_nodes, shifted, rays.view(orc.RAY_DTYPE), nthreads=8)
         assert_hits_equal(got, ref, f"after refit {step}")
         assert got.tobytes() != first.tobytes()
+
+
+def leaf_tree(tris):
+    """One root leaf over all triangles."""
+    nodes = np.zeros(2, B.NODE_DTYPE)
+    v = tris.reshape(-1, 3)
+    nodes["bmin"][0], nodes["bmax"][0], nodes["count"][0] = v.min(0), v.max(0), tris.shape[0]
+    return nodes, 2
+
+
+@pytest.mark.parametrize("mesh,n", [("soup", 1), ("soup", 17), ("soup", 65536), ("soup", 65537), ("sphere", 7501),
+                                    ("sphere", 65539), ("repeated", 4099), ("small", 65537), ("single", 3001)])
+def test_trees_with_large_leaves(ctx, orc, mesh, n):
+    """A group of 16 or 8 lanes a ray (by ray count and how uneven the leaves
+    are) gives the oracle's hits bit for bit: the reference builder's trees of
+    a soup (uneven leaves) and a sphere (even ones), a leaf in which every
+    triangle occurs five times (the first of equal distances), leaves below 64
+    triangles, and a leaf of one lane's worth; rays with a bound, without one,
+    with t = +inf and NaN, and with zero direction components."""
+    if mesh in ("soup", "small"):
+        tris = scenes.triangle_soup(3000 if mesh == "soup" else 300, seed=31)
+    elif mesh == "sphere":
+        tris = scenes.icosphere(12, radius=4.0, seed=5)
+    else:
+        tris = scenes.triangle_soup(40 if mesh == "repeated" else 7, seed=32)
+    if mesh in ("repeated", "single"):
+        tris = np.ascontiguousarray(np.tile(tris, (5 if mesh == "repeated" else 1, 1)))
+        nodes, used = leaf_tree(tris)
+    else:
+        nodes, used, tris = orc.bvh_build(tris, True, 0)
+    bvh = upload(ctx, nodes, used, tris)
+    rays = random_rays(n, 77)
+    rays["d"][5::11, 0] = 0.0
+    rays["d"][6::13, 1:] = 0.0
+    rays["tmax"][3::7] = np.inf
+    rays["tmax"][10::31] = np.nan
+    ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+    assert_hits_equal(bvh.intersect(rays), ref, f"{mesh} {n}")
+    assert n < 100 or (ref["prim"] != B.MISS).sum() > 5
+    bvh.close()
