@@ -49,6 +49,8 @@ struct BatchScene {
 struct BatchBlas {
     bvht_node* nodes;
     const float* tris;
+    const uint32_t* level;
+    const uint32_t* chunks;
 };
 
 __device__ __forceinline__ uint32_t upper_index(const uint32_t* prefix, uint32_t n, uint32_t x)
@@ -63,6 +65,16 @@ __device__ __forceinline__ uint32_t upper_index(const uint32_t* prefix, uint32_t
             hi = mid;
     }
     return lo;
+}
+
+// Refit inside the chunks of every BLAS of the batch: entries are (BLAS,
+// chunk) pairs, one workgroup each.
+__global__ __launch_bounds__(kChunkWG) void k_batch_refit_chunks(const BatchBlas* __restrict__ blases,
+                                                                 const uint2* __restrict__ entries)
+{
+    const uint2 e = entries[blockIdx.x];
+    const BatchBlas bb = blases[e.x];
+    refit_chunk(bb.nodes, bb.tris, bb.level, bb.chunks[e.y], bb.chunks[e.y + 1]);
 }
 
 // One tree level of every BLAS of the batch: entries are (BLAS, node) pairs.
@@ -214,7 +226,9 @@ struct bvht_batch_s {
     std::vector<bvht_blas> blases;
     BatchScene* d_scenes = nullptr;
     BatchBlas* d_blases = nullptr;
-    uint2* d_refit = nullptr;           // (BLAS, node) of every used node, grouped by level
+    uint2* d_refit = nullptr;           // (BLAS, node) of the nodes that cross chunks, grouped by level
+    uint2* d_refit_chunks = nullptr;    // (BLAS, chunk) of every chunk
+    uint32_t n_refit_chunks = 0;
     uint2* d_refit_big = nullptr;       // (BLAS, leaf) of every big leaf
     uint32_t n_refit_big = 0;
     std::vector<uint32_t> refit_off;     // level L occupies [refit_off[L], refit_off[L+1])
@@ -246,6 +260,7 @@ void batch_free(bvht_batch b)
     (void)hipFree(b->d_scenes);
     (void)hipFree(b->d_blases);
     (void)hipFree(b->d_refit);
+    (void)hipFree(b->d_refit_chunks);
     (void)hipFree(b->d_refit_big);
     (void)hipFree(b->d_obj_prefix);
     (void)hipFree(b->d_items);
@@ -312,20 +327,27 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
                 b->blases.push_back(bl);
     }
     std::vector<BatchBlas> hb(b->blases.size());
+    std::vector<uint2> chunks;
     uint32_t max_depth = 0;
     for (size_t k = 0; k < b->blases.size(); ++k) {
         bvht_blas bl = b->blases[k];
         hb[k].nodes = bl->d_nodes;
         hb[k].tris = bl->d_tris;
+        hb[k].level = bl->d_level;
+        hb[k].chunks = bl->d_chunks;
+        for (uint32_t c = 0; c < chunk_count(bl->nodes_used); ++c)
+            chunks.push_back(make_uint2((uint32_t)k, c));
         max_depth = std::max(max_depth, bl->depth);
     }
-    // combined level table: level L lists (BLAS, node) for every BLAS's level-L nodes
+    b->n_refit_chunks = (uint32_t)chunks.size();
+    // combined level table: level L lists (BLAS, node) for every BLAS's level-L
+    // nodes that cross chunk boundaries
     std::vector<std::vector<uint32_t>> orders(b->blases.size());
     b->refit_off.assign(max_depth + 1, 0);
     for (size_t k = 0; k < b->blases.size(); ++k) {
         bvht_blas bl = b->blases[k];
         orders[k].resize(bl->level_off.back());
-        if (hipMemcpy(orders[k].data(), bl->d_level_order, sizeof(uint32_t) * orders[k].size(),
+        if (!orders[k].empty() && hipMemcpy(orders[k].data(), bl->d_level_order, sizeof(uint32_t) * orders[k].size(),
                       hipMemcpyDeviceToHost) != hipSuccess) {
             delete b;
             return set_error(BVHT_EDEVICE, "batch: level table download failed");
@@ -361,6 +383,7 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
     bool ok = hipMalloc(&b->d_scenes, sizeof(BatchScene) * n_scenes) == hipSuccess &&
               hipMalloc(&b->d_blases, sizeof(BatchBlas) * hb.size()) == hipSuccess &&
               hipMalloc(&b->d_refit, sizeof(uint2) * std::max<size_t>(entries.size(), 1)) == hipSuccess &&
+              hipMalloc(&b->d_refit_chunks, sizeof(uint2) * chunks.size()) == hipSuccess &&
               hipMalloc(&b->d_refit_big, sizeof(uint2) * std::max<size_t>(big.size(), 1)) == hipSuccess &&
               hipMalloc(&b->d_obj_prefix, sizeof(uint32_t) * obj_prefix.size()) == hipSuccess &&
               hipMalloc(&b->d_items, sizeof(uint32_t) * (n_scenes + 1)) == hipSuccess &&
@@ -373,7 +396,9 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
     hipStream_t st = ctx->stream;
     if (hipMemcpyAsync(b->d_scenes, hs.data(), sizeof(BatchScene) * n_scenes, hipMemcpyHostToDevice, st) ||
         hipMemcpyAsync(b->d_blases, hb.data(), sizeof(BatchBlas) * hb.size(), hipMemcpyHostToDevice, st) ||
-        hipMemcpyAsync(b->d_refit, entries.data(), sizeof(uint2) * entries.size(), hipMemcpyHostToDevice, st) ||
+        (!entries.empty() &&
+         hipMemcpyAsync(b->d_refit, entries.data(), sizeof(uint2) * entries.size(), hipMemcpyHostToDevice, st)) ||
+        hipMemcpyAsync(b->d_refit_chunks, chunks.data(), sizeof(uint2) * chunks.size(), hipMemcpyHostToDevice, st) ||
         (!big.empty() &&
          hipMemcpyAsync(b->d_refit_big, big.data(), sizeof(uint2) * big.size(), hipMemcpyHostToDevice, st)) ||
         hipMemcpyAsync(b->d_obj_prefix, obj_prefix.data(), sizeof(uint32_t) * obj_prefix.size(),
@@ -406,8 +431,11 @@ int32_t bvht_batch_refit(bvht_ctx ctx, bvht_batch b)
     if (b->n_refit_big)
         hipLaunchKernelGGL(k_batch_refit_big, dim3(nblk(b->n_refit_big, 4)), dim3(256), 0, ctx->stream, b->d_blases,
                            b->d_refit_big, b->n_refit_big);
-    // a level of more than kRunWG entries gets a launch of its own; runs of
-    // consecutive smaller levels share one single-workgroup launch
+    hipLaunchKernelGGL(k_batch_refit_chunks, dim3(b->n_refit_chunks), dim3(kChunkWG), 0, ctx->stream, b->d_blases,
+                       b->d_refit_chunks);
+    // what crosses chunk boundaries: a level of more than kRunWG entries gets a
+    // launch of its own; runs of consecutive smaller levels share one
+    // single-workgroup launch
     EntryRun run{};
     auto flush = [&]() {
         if (run.levels)

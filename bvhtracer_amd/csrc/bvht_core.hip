@@ -185,7 +185,9 @@ __global__ __launch_bounds__(256) void k_levels(uint32_t nodes_used, const uint3
         atomicMax(depth, m);
 }
 
-// Per-level node counts and the level-grouped node order.  Levels below
+// Per-level counts and the level-grouped order of the nodes that refit_chunk
+// leaves (bit 31 of their level clear); the others are counted in hist[depth].
+// Levels below
 // kLevelsLds are counted in LDS first, so each workgroup issues one global
 // atomic per level instead of one per node (a few dozen counters shared by
 // millions of nodes serialise otherwise); deeper levels (degenerate trees)
@@ -198,23 +200,32 @@ constexpr uint32_t kLevelsLds = 64;
 __global__ void k_level_hist(uint32_t nodes_used, uint32_t depth, const uint32_t* __restrict__ level,
                              uint32_t* __restrict__ hist)
 {
-    __shared__ uint32_t sh[kLevelsLds];
+    __shared__ uint32_t sh[kLevelsLds], sh_in;
     for (uint32_t i = threadIdx.x; i < kLevelsLds; i += blockDim.x)
         sh[i] = 0;
+    if (threadIdx.x == 0)
+        sh_in = 0;
     __syncthreads();
+    uint32_t in = 0;
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nodes_used; k += gridDim.x * blockDim.x) {
         if (k == 1)
             continue;
         uint32_t L = level[k];
-        if (L < kLevelsLds && L < depth)
+        if (L & kInChunk)
+            in += (L & ~kInChunk) < depth;
+        else if (L < kLevelsLds && L < depth)
             atomicAdd(&sh[L], 1u);
         else if (L < depth)
             atomicAdd(&hist[L], 1u);
     }
+    if (in)
+        atomicAdd(&sh_in, in);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < kLevelsLds; i += blockDim.x)
         if (sh[i])
             atomicAdd(&hist[i], sh[i]);
+    if (threadIdx.x == 0 && sh_in)
+        atomicAdd(&hist[depth], sh_in);
 }
 
 __global__ void k_level_scatter(uint32_t nodes_used, uint32_t depth, const uint32_t* __restrict__ level,
@@ -276,6 +287,35 @@ __global__ __launch_bounds__(256) void k_refit_big_leaves(bvht_node* __restrict_
     uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (w < count)
         refit_big_leaf(nodes, tris, list[w], threadIdx.x & 63u);
+}
+
+// chunks[c] = first node of chunk c, chunks[chunk count] = nodes_used; a wave
+// per chunk, before the marks go into the levels.
+__global__ __launch_bounds__(256) void k_chunk_starts(const uint32_t* __restrict__ level, uint32_t nodes_used,
+                                                      uint32_t count, uint32_t* __restrict__ chunks)
+{
+    const uint32_t c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (c > count)
+        return;
+    const uint32_t at = c == count ? nodes_used : chunk_start(level, nodes_used, c, lane);
+    if (lane == 0)
+        chunks[c] = at;
+}
+
+__global__ __launch_bounds__(kChunkWG) void k_mark_chunks(const bvht_node* __restrict__ nodes,
+                                                          const uint32_t* __restrict__ chunks,
+                                                          uint32_t* __restrict__ level)
+{
+    mark_chunk(nodes, chunks[blockIdx.x], chunks[blockIdx.x + 1], level);
+}
+
+// Bvh::refit inside the chunks (see refit_chunk); the level passes follow.
+__global__ __launch_bounds__(kChunkWG) void k_refit_chunks(bvht_node* __restrict__ nodes,
+                                                           const float* __restrict__ tris,
+                                                           const uint32_t* __restrict__ level,
+                                                           const uint32_t* __restrict__ chunks)
+{
+    refit_chunk(nodes, tris, level, chunks[blockIdx.x], chunks[blockIdx.x + 1]);
 }
 
 // Bvh::refit, one tree level (see refit_node).
@@ -1285,22 +1325,21 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
 {
     bvht_ctx ctx = b->ctx;
     hipStream_t st = ctx->stream;
-    int32_t rc = fill_u32(ctx, b->d_parent, BVHT_MISS, b->node_count);
-    if (rc)
-        return rc;
     uint32_t nb = blocks_for(b->nodes_used, 256);
-    hipLaunchKernelGGL(k_parents, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, b->d_parent);
-    // scratch: [0] depth, then the per-level counts, then the big-leaf count
-    // and the widest leaf
-    rc = ensure_scratch(ctx, sizeof(uint32_t) * (2 * (size_t)b->nodes_used + 4));
+    // scratch: [0] depth, then the per-level counts, the count of the nodes
+    // inside chunks, the big-leaf count and the widest leaf
+    int32_t rc = ensure_scratch(ctx, sizeof(uint32_t) * (2 * (size_t)b->nodes_used + 4));
     if (rc)
         return rc;
     uint32_t* d_depth = static_cast<uint32_t*>(ctx->scratch);
     uint32_t depth = known_depth;
     if (depth == 0) {
-        rc = fill_u32(ctx, d_depth, 0, 1);
+        rc = fill_u32(ctx, b->d_parent, BVHT_MISS, b->node_count);
+        if (!rc)
+            rc = fill_u32(ctx, d_depth, 0, 1);
         if (rc)
             return rc;
+        hipLaunchKernelGGL(k_parents, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, b->d_parent);
         hipLaunchKernelGGL(k_levels, dim3(nb), dim3(256), 0, st, b->nodes_used, b->d_parent, b->d_level, d_depth);
         BVHT_HIP(hipGetLastError());
         BVHT_HIP(hipMemcpyAsync(&depth, d_depth, 4, hipMemcpyDeviceToHost, st));
@@ -1310,10 +1349,16 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
         return set_error(BVHT_EDEVICE, "BLAS topology: depth %u out of range", depth);
     b->depth = depth;
     uint32_t* hist = d_depth + 1;
-    uint32_t* big = hist + depth;  // big-leaf count, widest leaf
-    rc = fill_u32(ctx, hist, 0, depth + 2);
+    uint32_t* big = hist + depth + 1;  // big-leaf count, widest leaf
+    rc = fill_u32(ctx, hist, 0, depth + 3);
     if (rc)
         return rc;
+    // (a tree with shared nodes keeps to the level passes)
+    const uint32_t n_chunks = chunk_count(b->nodes_used);
+    hipLaunchKernelGGL(k_chunk_starts, dim3(blocks_for(n_chunks + 1, 4)), dim3(256), 0, st, b->d_level, b->nodes_used,
+                       n_chunks, b->d_chunks);
+    if (b->one_parent)
+        hipLaunchKernelGGL(k_mark_chunks, dim3(n_chunks), dim3(kChunkWG), 0, st, b->d_nodes, b->d_chunks, b->d_level);
     uint32_t nb_levels = std::min<uint32_t>(nb, 512);
     hipLaunchKernelGGL(k_level_hist, dim3(nb_levels), dim3(256), 0, st, b->nodes_used, depth, b->d_level, hist);
     // big leaves: counted here, listed below; and whether every node fits a
@@ -1321,21 +1366,21 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     hipLaunchKernelGGL(k_big_leaves, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, big, nullptr, big + 1,
                        mean_leaf(b) >= kGroupLeaf ? 1u : 64u);
     BVHT_HIP(hipGetLastError());
-    std::vector<uint32_t> h(depth + 2);
-    BVHT_HIP(hipMemcpyAsync(h.data(), hist, sizeof(uint32_t) * (depth + 2), hipMemcpyDeviceToHost, st));
+    std::vector<uint32_t> h(depth + 3);
+    BVHT_HIP(hipMemcpyAsync(h.data(), hist, sizeof(uint32_t) * (depth + 3), hipMemcpyDeviceToHost, st));
     BVHT_HIP(hipStreamSynchronize(st));
     b->level_off.assign(depth + 1, 0);
     for (uint32_t L = 0; L < depth; ++L)
         b->level_off[L + 1] = b->level_off[L] + h[L];
-    if (b->level_off[depth] + 1 != b->nodes_used && !(b->nodes_used == 1))
-        return set_error(BVHT_EDEVICE, "BLAS topology: %u nodes grouped, %u expected", b->level_off[depth],
+    if (b->level_off[depth] + h[depth] + 1 != b->nodes_used && !(b->nodes_used == 1))
+        return set_error(BVHT_EDEVICE, "BLAS topology: %u nodes grouped, %u expected", b->level_off[depth] + h[depth],
                          b->nodes_used - 1);
     BVHT_HIP(hipMemcpyAsync(hist, b->level_off.data(), sizeof(uint32_t) * depth, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_level_scatter, dim3(nb_levels), dim3(256), 0, st, b->nodes_used, depth, b->d_level, hist,
                        b->d_level_order);
     BVHT_HIP(hipGetLastError());
-    uint32_t nbig = h[depth];
-    b->widest_leaf = h[depth + 1];
+    uint32_t nbig = h[depth + 1];
+    b->widest_leaf = h[depth + 2];
     b->packed_stack = b->widest_leaf < 64 && b->nodes_used <= kPackMask + 1u && b->n_tris <= kPackMask + 1u;
     (void)hipFree(b->d_big_leaves);
     b->d_big_leaves = nullptr;
@@ -1354,14 +1399,17 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     return BVHT_OK;
 }
 
-// Bvh::refit, deepest level first: a level of more than kRunWG nodes gets a
-// launch of its own; runs of consecutive smaller levels (the top of the tree
-// and sparse deep levels) share one single-workgroup launch.
+// Bvh::refit: the chunks, then the branches that cross chunk boundaries,
+// deepest level first: a level of more than kRunWG of them gets a launch of its
+// own; runs of consecutive smaller levels share one single-workgroup launch.
+// 2 launches for 82k triangles, where level passes over all nodes took 10.
 int32_t launch_refit(bvht_ctx ctx, bvht_blas blas)
 {
     if (blas->n_big_leaves)
         hipLaunchKernelGGL(k_refit_big_leaves, dim3(blocks_for(blas->n_big_leaves, 4)), dim3(256), 0, ctx->stream,
                            blas->d_nodes, blas->d_tris, blas->d_big_leaves, blas->n_big_leaves);
+    hipLaunchKernelGGL(k_refit_chunks, dim3(chunk_count(blas->nodes_used)), dim3(kChunkWG), 0, ctx->stream,
+                       blas->d_nodes, blas->d_tris, blas->d_level, blas->d_chunks);
     LevelRun run{};
     auto flush = [&]() {
         if (run.levels)
@@ -1416,6 +1464,22 @@ static int32_t validate_nodes(const bvht_node* nodes, uint32_t node_count, uint3
     return BVHT_OK;
 }
 
+// Whether every node has at most one parent, as in every tree this library
+// builds (then a child is exactly one level below its parent).
+static bool one_parent_each(const bvht_node* nodes, uint32_t nodes_used)
+{
+    std::vector<bool> seen(nodes_used, false);
+    for (uint32_t k = 0; k < nodes_used; ++k) {
+        if (k == 1 || nodes[k].count > 0)
+            continue;
+        const uint32_t lf = nodes[k].left_first;
+        if (seen[lf] || seen[lf + 1])
+            return false;
+        seen[lf] = seen[lf + 1] = true;
+    }
+    return true;
+}
+
 constexpr size_t kBlasPoolBytes = size_t(1) << 30;
 constexpr size_t kBlasPoolEntries = 32;
 
@@ -1462,7 +1526,8 @@ int32_t blas_alloc(bvht_ctx ctx, uint32_t n, uint32_t node_count, bvht_blas* out
     b->d_parent = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)node_count));
     b->d_level = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)node_count));
     b->d_level_order = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)node_count));
-    bool ok = b->d_nodes && b->d_tris && b->d_parent && b->d_level && b->d_level_order;
+    b->d_chunks = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (chunk_count(node_count) + 1)));
+    bool ok = b->d_nodes && b->d_tris && b->d_parent && b->d_level && b->d_level_order && b->d_chunks;
     if (!ok) {
         bvht_blas_destroy(b);
         return set_error(BVHT_ENOMEM, "device allocation for a BLAS of %u triangles failed", n);
@@ -1930,6 +1995,7 @@ int32_t bvht_blas_upload(bvht_ctx ctx, const bvht_node* nodes, uint32_t node_cou
     if (rc)
         return rc;
     b->nodes_used = nodes_used;
+    b->one_parent = one_parent_each(nodes, nodes_used);
     rc = host_to_device(ctx, b->d_nodes, nodes, sizeof(bvht_node) * (size_t)node_count);
     if (!rc)
         rc = host_to_device(ctx, b->d_tris, tris, sizeof(float) * 9 * (size_t)n);
@@ -2024,6 +2090,7 @@ int32_t bvht_blas_destroy(bvht_blas b)
     blas_buffer_release(c, b->d_parent, sizeof(uint32_t) * nc);
     blas_buffer_release(c, b->d_level, sizeof(uint32_t) * nc);
     blas_buffer_release(c, b->d_level_order, sizeof(uint32_t) * nc);
+    blas_buffer_release(c, b->d_chunks, sizeof(uint32_t) * (chunk_count((uint32_t)nc) + 1));
     (void)hipFree(b->d_big_leaves);
     (void)hipFree(b->d_attr_normals);
     (void)hipFree(b->d_attr_tex);

@@ -112,12 +112,14 @@ struct bvht_blas_s {
     bvht_node* d_nodes = nullptr;
     float* d_tris = nullptr;  // 9 floats per triangle, build order
     uint32_t* d_perm = nullptr;  // input index of the triangle at each build position (GPU builds only)
-    uint32_t* d_parent = nullptr;       // parent of each used node (root: 0xFFFFFFFF)
-    uint32_t* d_level = nullptr;        // depth of each used node (root 0; dummy node 1: 0xFFFFFFFF)
-    uint32_t* d_level_order = nullptr;  // used nodes except the dummy, grouped by level
+    uint32_t* d_parent = nullptr;       // parent of each used node of an uploaded tree (root: 0xFFFFFFFF)
+    uint32_t* d_level = nullptr;        // depth of each used node (root 0; dummy node 1: 0xFFFFFFFF), bit 31: refit_chunk's
+    uint32_t* d_level_order = nullptr;  // the nodes refit_chunk leaves, grouped by level
+    uint32_t* d_chunks = nullptr;       // first node of each refit chunk, then nodes_used
     std::vector<uint32_t> level_off;    // level L occupies [level_off[L], level_off[L+1]) of d_level_order
     uint32_t* d_big_leaves = nullptr;   // leaves with more than kBigLeaf triangles (refit a wave each)
     uint32_t n_big_leaves = 0;
+    bool one_parent = true;     // no node has two parents (an uploaded tree's may)
     uint32_t widest_leaf = 0;   // triangles of the largest leaf (0 if below 64 and leaves are small on average)
     bool packed_stack = false;  // every node fits a packed stack entry (see bvht_trace.hpp)
     // shading attributes (bvht_blas_set_attributes)

@@ -8,7 +8,7 @@ import pytest
 
 import bvhtracer_amd as B
 from bvhtracer_amd import scenes
-from helpers import assert_hits_equal, assert_nodes_equal, upload
+from helpers import assert_hits_equal, assert_nodes_equal, comb_tree, upload
 
 pytestmark = pytest.mark.gpu
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -239,4 +239,53 @@ def test_build_mid_sizes_match_oracle(ctx, orc, freq, mode, max_leaf):
     assert g_tris.tobytes() == perm.tobytes()
     assert m.tobytes() == perm.tobytes()  # the caller's array holds the permuted triangles
     assert bvh.depth() == orc.bvh_depth(nodes)
+    bvh.close()
+
+
+def breadth_first(nodes, used):
+    """The same tree with its child pairs numbered level by level."""
+    out = np.zeros_like(nodes)
+    out[0] = nodes[0]
+    queue, nxt = [(0, 0)], 2
+    for old, new in queue:
+        out[new] = nodes[old]
+        if nodes[old]["count"] == 0:
+            lf = int(nodes[old]["left_first"])
+            out[new]["left_first"] = nxt
+            queue += [(lf, nxt), (lf + 1, nxt + 1)]
+            nxt += 2
+    assert nxt == used
+    return out
+
+
+@pytest.mark.parametrize("tree", ["soup1", "soup2", "soup511", "soup512", "soup513", "soup1024", "soup5000", "sphere24500",
+                                  "breadth5000", "comb3000", "reference5000", "shared"])
+def test_refit_across_chunk_boundaries(ctx, orc, tree):
+    """Refit takes chunks of 1,024 nodes in LDS and passes of the branches that
+    cross them: trees around one and several chunks, a tree numbered breadth
+    first (nearly every branch crosses), a comb of 3,000 levels, big leaves,
+    and a tree with a pair under two parents (no chunks); every box equals the
+    oracle's reverse sweep, twice in a row and from other vertices."""
+    kind, n = tree.rstrip("0123456789"), int(tree.lstrip("abcdefghijklmnopqrstuvwxyz") or 0)
+    if kind == "comb":
+        nodes, used, tris = comb_tree(n)
+    elif kind == "shared":
+        nodes, used, tris = comb_tree(3)
+        nodes = np.concatenate([nodes[:4], nodes[4:6], nodes[:2]])
+        nodes[3]["left_first"], nodes[3]["count"] = 4, 0
+        assert used == 6
+    else:
+        mesh = scenes.icosphere(35, seed=9) if kind == "sphere" else scenes.triangle_soup(n, seed=n)
+        nodes, used, tris = orc.bvh_build(mesh, kind == "reference", 1)
+        if kind == "breadth":
+            nodes = breadth_first(nodes, used)
+    bvh = upload(ctx, nodes, used, tris)
+    want = nodes.copy()
+    for frame in (3, 3, 17):
+        moved = scenes.deform_wave(tris, frame, amp=0.7)
+        orc.bvh_refit(want, used, moved)
+        bvh.refit(moved)
+        got, g_used, _ = bvh.download()
+        assert g_used == used
+        assert_nodes_equal(got, want, used)
     bvh.close()
