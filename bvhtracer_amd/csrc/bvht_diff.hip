@@ -297,11 +297,13 @@ __global__ __launch_bounds__(WG) void k_trace_forward(const float4* __restrict__
     }
     image[i] = make_float2(depth, shade);
     // lane 0 is always a ray of the group (group * 64 < n)
-    if ((threadIdx.x & 63) == 0) {
+    if (cost && (threadIdx.x & 63) == 0) {
         uint64_t dt = (uint64_t)wall_clock64() - t0;
         cost[group] = dt > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)dt;
     }
 }
+
+constexpr uint32_t kSchedGroups = 4096;
 
 typedef void (*forward_fn)(const float4*, const float*, const uint32_t*, const float*, Rows, V3, const bvht_ray*,
                            uint32_t, bvht_hit*, float2*, uint32_t*, uint32_t, uint32_t*, const uint32_t*,
@@ -514,10 +516,16 @@ __global__ __launch_bounds__(kAdjWG) void k_trace_adjoint(
 // t + kFinWG, ... for all components at once (each block's partials are one
 // 128-byte row), then a butterfly within each wave and the waves in order.
 constexpr int kFinWG = 1024;
+struct AdjFinish {
+    const double* partials;
+    uint32_t nblocks;  // 0: not in this launch
+    int accumulate;
+    float* grad_minv;
+    double* loss;
+};
 
-__global__ __launch_bounds__(kFinWG) void k_adjoint_finish(const double* __restrict__ partials, uint32_t nblocks,
-                                                           int accumulate, float* __restrict__ grad_minv,
-                                                           double* __restrict__ loss)
+__device__ __forceinline__ void adjoint_finish(const double* __restrict__ partials, uint32_t nblocks, int accumulate,
+                                               float* __restrict__ grad_minv, double* __restrict__ loss)
 {
     __shared__ double red[kFinWG / 64][kRed];
     double acc[kRed];
@@ -567,9 +575,12 @@ __global__ __launch_bounds__(kFinWG) void k_adjoint_finish(const double* __restr
 // a bucket comes from the atomics; k_adj_triangles sorts it.
 __global__ __launch_bounds__(256) void k_adj_place(const uint32_t* __restrict__ rec_key, uint32_t slots,
                                                     const uint32_t* __restrict__ tri_off,
-                                                    uint32_t* __restrict__ tri_cur, uint32_t* __restrict__ bucket)
+                                                    uint32_t* __restrict__ tri_cur, uint32_t* __restrict__ bucket,
+                                                    uint32_t* __restrict__ n_big)
 {
     uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i == 0)
+        *n_big = 0;  // the list of k_adj_triangles, which follows
     if (i >= slots)
         return;
     uint32_t t = rec_key[i];
@@ -630,21 +641,30 @@ __global__ __launch_bounds__(256) void k_adj_triangles(uint32_t nt, uint32_t* __
     tri_cur[t] = 0u;
 }
 
-// Triangles with more than kAdjSmall records (at most kAdjBigMax): one
-// workgroup per triangle, the gridded workgroups taking the listed triangles
-// in turn.  The bucket is bitonic-sorted in LDS, thread k sums sorted
+// The first workgroup sums the blocks' partials (adjoint_finish), which only
+// k_trace_adjoint writes: beside the triangles' sums instead of after them
+// (15 us of its own launch for 2M rays).  The others: triangles with more than
+// kAdjSmall records (at most kAdjBigMax), one workgroup per triangle, the
+// gridded workgroups taking the listed triangles in turn.  The bucket is bitonic-sorted in LDS, thread k sums sorted
 // records [k c, (k+1) c) in order (c = ceil(cnt / kAdjBigWG)), the partial
 // sums are added by a butterfly within each wave and the waves in order.
 __global__ __launch_bounds__(kAdjBigWG) void k_adj_big(const uint32_t* __restrict__ big,
                                                       const uint32_t* __restrict__ n_big,
                                                       uint32_t* __restrict__ tri_off, uint32_t* __restrict__ tri_cur,
                                                       const uint32_t* __restrict__ bucket,
-                                                      const float* __restrict__ rec_val, float* __restrict__ tgrad)
+                                                      const float* __restrict__ rec_val, float* __restrict__ tgrad,
+                                                      AdjFinish fin)
 {
+    static_assert(kFinWG == kAdjBigWG, "adjoint_finish runs in a workgroup of k_adj_big");
     __shared__ uint32_t keys[kAdjBigMax];
     __shared__ float wsum[kAdjBigWG / 64][9];
+    if (blockIdx.x == 0) {
+        if (fin.nblocks)
+            adjoint_finish(fin.partials, fin.nblocks, fin.accumulate, fin.grad_minv, fin.loss);
+        return;
+    }
     uint32_t nb = *n_big;
-    for (uint32_t q = blockIdx.x; q < nb; q += gridDim.x) {
+    for (uint32_t q = blockIdx.x - 1; q < nb; q += gridDim.x - 1) {
         uint32_t t = big[q];
         uint32_t cnt = tri_cur[t];
         const uint32_t* b = bucket + tri_off[t];
@@ -957,7 +977,11 @@ extern "C" int32_t bvht_trace_forward(bvht_ctx ctx, bvht_mesh mesh, const float*
     if (!fn)
         return set_error(BVHT_EINVAL, "no forward kernel for workgroup %d, LDS depth %d", wg, lds);
     uint32_t groups = nblk(n, 64);
-    if (groups > mesh->sched_cap) {
+    // A launch whose waves are all resident at once (7 a SIMD) has no order to
+    // choose: no durations, no order, four launches fewer (16k rays 65 -> 57 us,
+    // 250k 153 -> 136; 500k, where the order begins to pay, 166 with it).
+    const bool ordered = groups > kSchedGroups;
+    if (ordered && groups > mesh->sched_cap) {
         BVHT_REQUIRE(ctx->live_graphs == 0 && !ctx->capturing,
                      "the forward schedule must grow to %u groups, but a graph captured on this context holds its "
                      "address: make one eager call of the largest ray count first", groups);
@@ -973,12 +997,15 @@ extern "C" int32_t bvht_trace_forward(bvht_ctx ctx, bvht_mesh mesh, const float*
         mesh->sched_cap = groups;
     }
     // the schedule made by the last forward over the same number of rays
-    const uint32_t* sched = mesh->sched_n == n ? mesh->d_sched : nullptr;
+    const uint32_t* sched = ordered && mesh->sched_n == n ? mesh->d_sched : nullptr;
     hipLaunchKernelGGL(fn, dim3(nblk(groups, wg / 64)), dim3(wg), 0, ctx->stream,
                        reinterpret_cast<const float4*>(b->d_nodes), b->d_tris, mesh->d_vid, mesh->d_normals,
                        rows_of(minv), V3{light[0], light[1], light[2]}, d_rays, n, d_hits,
                        reinterpret_cast<float2*>(d_image), spill, need, ctx->d_status, sched,
-                       sched_units(mesh->d_bins), mesh->d_cost);
+                       sched ? sched_units(mesh->d_bins) : nullptr, ordered ? mesh->d_cost : nullptr);
+    BVHT_HIP(hipGetLastError());
+    if (!ordered)
+        return BVHT_OK;
     // the schedule for the next forward: longest groups first
     int32_t rc = launch_longest_first(ctx, mesh->d_cost, groups, mesh->d_bins, mesh->d_sched);
     if (rc)
@@ -1028,23 +1055,19 @@ extern "C" int32_t bvht_trace_adjoint(bvht_ctx ctx, bvht_mesh mesh, const float*
                            rec_key, rec_val, mesh->d_poff, partials + 16 * (size_t)(first / kAdjWG));
         launch_scan(ctx, mesh->d_poff, nt, mesh->d_psums, nullptr);
         hipLaunchKernelGGL(k_adj_place, dim3(nblk(slots, 256)), dim3(256), 0, ctx->stream, rec_key, slots,
-                           mesh->d_poff, mesh->d_pcur, bucket);
-        rc = fill_u32(ctx, mesh->d_nbig, 0u, 1);
-        if (rc)
-            return rc;
+                           mesh->d_poff, mesh->d_pcur, bucket, mesh->d_nbig);
         hipLaunchKernelGGL(k_adj_triangles, dim3(nblk(nt, 256)), dim3(256), 0, ctx->stream, nt, mesh->d_poff,
                            mesh->d_pcur, bucket, rec_val, mesh->d_tgrad, mesh->d_big, mesh->d_nbig);
-        hipLaunchKernelGGL(k_adj_big, dim3(std::min<uint32_t>(nt, 64)), dim3(kAdjBigWG), 0, ctx->stream,
-                           mesh->d_big, mesh->d_nbig, mesh->d_poff, mesh->d_pcur, bucket, rec_val, mesh->d_tgrad);
+        const bool last = n - first <= kAdjPass;
+        hipLaunchKernelGGL(k_adj_big, dim3(1 + std::min<uint32_t>(nt, 64)), dim3(kAdjBigWG), 0, ctx->stream,
+                           mesh->d_big, mesh->d_nbig, mesh->d_poff, mesh->d_pcur, bucket, rec_val, mesh->d_tgrad,
+                           AdjFinish{partials, last ? nb : 0u, (int)accumulate, d_grad_minv, d_loss});
         hipLaunchKernelGGL(k_adj_vertices, dim3(nblk(mesh->n_vertices, 256)), dim3(256), 0, ctx->stream,
                            mesh->n_vertices, mesh->d_vt_off, mesh->d_vt_idx, mesh->d_tgrad,
                            (int)(accumulate || first > 0), d_grad_vertices);
         BVHT_HIP(hipGetLastError());
-        if (n - first <= kAdjPass)
+        if (last)
             break;
     }
-    hipLaunchKernelGGL(k_adjoint_finish, dim3(1), dim3(kFinWG), 0, ctx->stream, partials, nb, (int)accumulate,
-                       d_grad_minv, d_loss);
-    BVHT_HIP(hipGetLastError());
     return BVHT_OK;
 }
