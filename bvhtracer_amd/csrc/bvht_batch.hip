@@ -51,6 +51,7 @@ struct BatchBlas {
     const float* tris;
     const uint32_t* level;
     const uint32_t* chunks;
+    float4* wide;  // NULL: no wide records
 };
 
 __device__ __forceinline__ uint32_t upper_index(const uint32_t* prefix, uint32_t n, uint32_t x)
@@ -74,7 +75,21 @@ __global__ __launch_bounds__(kChunkWG) void k_batch_refit_chunks(const BatchBlas
 {
     const uint2 e = entries[blockIdx.x];
     const BatchBlas bb = blases[e.x];
-    refit_chunk(bb.nodes, bb.tris, bb.level, bb.chunks[e.y], bb.chunks[e.y + 1]);
+    refit_chunk(bb.nodes, bb.tris, bb.level, bb.chunks[e.y], bb.chunks[e.y + 1], bb.wide);
+}
+
+// The wide records of the BLASes that have them, after their refit: entries
+// are the same (BLAS, chunk) pairs.
+__global__ __launch_bounds__(kChunkWG) void k_batch_wide(const BatchBlas* __restrict__ blases,
+                                                         const uint2* __restrict__ entries)
+{
+    const uint2 e = entries[blockIdx.x];
+    const BatchBlas bb = blases[e.x];
+    if (!bb.wide)
+        return;
+    for (uint32_t k = bb.chunks[e.y] + threadIdx.x; k < bb.chunks[e.y + 1]; k += kChunkWG)
+        if (k != 1 && (bb.level[k] & 1u) == 0)
+            write_wide(reinterpret_cast<const float4*>(bb.nodes), bb.wide, k);
 }
 
 // One tree level of every BLAS of the batch: entries are (BLAS, node) pairs.
@@ -229,6 +244,7 @@ struct bvht_batch_s {
     uint2* d_refit = nullptr;           // (BLAS, node) of the nodes that cross chunks, grouped by level
     uint2* d_refit_chunks = nullptr;    // (BLAS, chunk) of every chunk
     uint32_t n_refit_chunks = 0;
+    bool any_wide = false;              // some BLAS has wide records
     uint2* d_refit_big = nullptr;       // (BLAS, leaf) of every big leaf
     uint32_t n_refit_big = 0;
     std::vector<uint32_t> refit_off;     // level L occupies [refit_off[L], refit_off[L+1])
@@ -335,6 +351,8 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
         hb[k].tris = bl->d_tris;
         hb[k].level = bl->d_level;
         hb[k].chunks = bl->d_chunks;
+        hb[k].wide = bl->d_wide;
+        b->any_wide = b->any_wide || bl->d_wide;
         for (uint32_t c = 0; c < chunk_count(bl->nodes_used); ++c)
             chunks.push_back(make_uint2((uint32_t)k, c));
         max_depth = std::max(max_depth, bl->depth);
@@ -459,6 +477,9 @@ int32_t bvht_batch_refit(bvht_ctx ctx, bvht_batch b)
             flush();
     }
     flush();
+    if (b->any_wide)
+        hipLaunchKernelGGL(k_batch_wide, dim3(b->n_refit_chunks), dim3(kChunkWG), 0, ctx->stream, b->d_blases,
+                           b->d_refit_chunks);
     BVHT_HIP(hipGetLastError());
     return BVHT_OK;
 }

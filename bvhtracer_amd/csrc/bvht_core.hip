@@ -263,13 +263,17 @@ __global__ void k_level_scatter(uint32_t nodes_used, uint32_t depth, const uint3
 
 // Leaves with more than kBigLeaf triangles: counted, then listed.  `widest`
 // (when given, 0 before) becomes the triangle count of the largest leaf of at
-// least `from` triangles.
+// least `from` triangles.  `wide` (when given): the wide records, written on
+// the way (a new tree's; used if it turns out packed).
 __global__ void k_big_leaves(const bvht_node* __restrict__ nodes, uint32_t nodes_used, uint32_t* __restrict__ counter,
-                             uint32_t* __restrict__ list, uint32_t* __restrict__ widest, uint32_t from)
+                             uint32_t* __restrict__ list, uint32_t* __restrict__ widest, uint32_t from,
+                             const uint32_t* __restrict__ level, float4* __restrict__ wide)
 {
     uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nodes_used || k == 1)
         return;
+    if (wide && (level[k] & 1u) == 0)
+        write_wide(reinterpret_cast<const float4*>(nodes), wide, k);
     uint32_t c = nodes[k].count;
     if (widest && c >= from && c > __hip_atomic_load(widest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
         atomicMax(widest, c);
@@ -304,8 +308,10 @@ __global__ __launch_bounds__(256) void k_chunk_starts(const uint32_t* __restrict
 
 __global__ __launch_bounds__(kChunkWG) void k_mark_chunks(const bvht_node* __restrict__ nodes,
                                                           const uint32_t* __restrict__ chunks,
-                                                          uint32_t* __restrict__ level)
+                                                          uint32_t* __restrict__ level, float4* __restrict__ wide)
 {
+    if (wide && blockIdx.x == 0 && threadIdx.x == 0)
+        *reinterpret_cast<uint32_t*>(wide) = 0;  // the records' mark
     mark_chunk(nodes, chunks[blockIdx.x], chunks[blockIdx.x + 1], level);
 }
 
@@ -313,9 +319,19 @@ __global__ __launch_bounds__(kChunkWG) void k_mark_chunks(const bvht_node* __res
 __global__ __launch_bounds__(kChunkWG) void k_refit_chunks(bvht_node* __restrict__ nodes,
                                                            const float* __restrict__ tris,
                                                            const uint32_t* __restrict__ level,
-                                                           const uint32_t* __restrict__ chunks)
+                                                           const uint32_t* __restrict__ chunks,
+                                                           float4* __restrict__ wide)
 {
-    refit_chunk(nodes, tris, level, chunks[blockIdx.x], chunks[blockIdx.x + 1]);
+    refit_chunk(nodes, tris, level, chunks[blockIdx.x], chunks[blockIdx.x + 1], wide);
+}
+
+// The wide record of every node at even depth, after the node boxes are final.
+__global__ __launch_bounds__(256) void k_wide(const float4* __restrict__ nodes, const uint32_t* __restrict__ level,
+                                              uint32_t nodes_used, float4* __restrict__ wide)
+{
+    uint32_t k = blockIdx.x * 256 + threadIdx.x;
+    if (k < nodes_used && k != 1 && (level[k] & 1u) == 0)
+        write_wide(nodes, wide, k);
 }
 
 // Bvh::refit, one tree level (see refit_node).
@@ -412,6 +428,24 @@ __global__ __launch_bounds__(256) void k_trace_group(const float4* __restrict__ 
     Stack<kGroupStack, kRays> st{(lds_u32*)(lds + threadIdx.x / G), spill + i, (size_t)n, cap, status};
     const BlasResult r = traverse_group<G>(nodes, tris, load_ray(rays, i), st);
     if (threadIdx.x % G == 0)
+        store_hit(hits, i, r.found, r.t, r.u, r.v, r.prim, 0);
+}
+
+// k_trace_blas with four lanes a ray (traverse_quad), `per` rays (1 to 16) a
+// wave.
+__global__ __launch_bounds__(64) void k_trace_quad(const float4* __restrict__ nodes, const float4* __restrict__ wide,
+                                                   const float* __restrict__ tris, const bvht_ray* __restrict__ rays,
+                                                   bvht_hit* __restrict__ hits, uint32_t n,
+                                                   const uint32_t* __restrict__ d_n, uint32_t* __restrict__ spill,
+                                                   uint32_t cap, uint32_t* __restrict__ status, uint32_t per)
+{
+    __shared__ uint32_t lds[kQuadLds * 64];
+    const uint32_t i = blockIdx.x * per + (threadIdx.x >> 2);
+    const uint32_t count = d_n ? min(*d_n, n) : n;
+    if ((threadIdx.x >> 2) >= per || i >= count)
+        return;
+    const BlasResult r = trace_quad(nodes, wide, tris, load_ray(rays, i), lds, spill + i, (size_t)n, cap, status);
+    if ((threadIdx.x & 3u) == 0)
         store_hit(hits, i, r.found, r.t, r.u, r.v, r.prim, 0);
 }
 
@@ -1317,6 +1351,19 @@ int32_t device_to_host_beside(bvht_ctx ctx, void* dst, const void* src, size_t b
     return device_to_host_on(ctx, cs, dst, src, bytes);
 }
 
+// Wide records are kept for packed trees of at most kWideTris triangles: every
+// refit writes them again (4 us, for 82k triangles 6), and on larger trees
+// launches small enough for traverse_quad are the rarer.
+constexpr uint32_t kWideTris = 1u << 16;
+static size_t wide_bytes(size_t node_count) { return 64 * node_count; }  // the last pair's record ends with them
+
+static void launch_wide(bvht_ctx ctx, bvht_blas b)
+{
+    if (b->d_wide)
+        hipLaunchKernelGGL(k_wide, dim3(blocks_for(b->nodes_used, 256)), dim3(256), 0, ctx->stream,
+                           reinterpret_cast<const float4*>(b->d_nodes), b->d_level, b->nodes_used, b->d_wide);
+}
+
 // Triangles of a leaf on average (nodes_used counts the dummy: two a leaf).
 static uint32_t mean_leaf(bvht_blas b) { return b->n_tris / std::max(1u, b->nodes_used / 2); }
 constexpr uint32_t kGroupLeaf = 6;  // mean from which leaf_group considers a group of lanes
@@ -1353,18 +1400,21 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     rc = fill_u32(ctx, hist, 0, depth + 3);
     if (rc)
         return rc;
+    if (b->one_parent && b->even_pairs && b->n_tris <= kWideTris && b->nodes_used > 2)
+        b->d_wide = static_cast<float4*>(blas_buffer(ctx, wide_bytes(b->node_count)));  // (none: no quads)
     // (a tree with shared nodes keeps to the level passes)
     const uint32_t n_chunks = chunk_count(b->nodes_used);
     hipLaunchKernelGGL(k_chunk_starts, dim3(blocks_for(n_chunks + 1, 4)), dim3(256), 0, st, b->d_level, b->nodes_used,
                        n_chunks, b->d_chunks);
     if (b->one_parent)
-        hipLaunchKernelGGL(k_mark_chunks, dim3(n_chunks), dim3(kChunkWG), 0, st, b->d_nodes, b->d_chunks, b->d_level);
+        hipLaunchKernelGGL(k_mark_chunks, dim3(n_chunks), dim3(kChunkWG), 0, st, b->d_nodes, b->d_chunks, b->d_level,
+                           b->d_wide);
     uint32_t nb_levels = std::min<uint32_t>(nb, 512);
     hipLaunchKernelGGL(k_level_hist, dim3(nb_levels), dim3(256), 0, st, b->nodes_used, depth, b->d_level, hist);
     // big leaves: counted here, listed below; and whether every node fits a
     // packed stack entry
     hipLaunchKernelGGL(k_big_leaves, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, big, nullptr, big + 1,
-                       mean_leaf(b) >= kGroupLeaf ? 1u : 64u);
+                       mean_leaf(b) >= kGroupLeaf ? 1u : 64u, b->d_level, b->d_wide);
     BVHT_HIP(hipGetLastError());
     std::vector<uint32_t> h(depth + 3);
     BVHT_HIP(hipMemcpyAsync(h.data(), hist, sizeof(uint32_t) * (depth + 3), hipMemcpyDeviceToHost, st));
@@ -1382,6 +1432,10 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     uint32_t nbig = h[depth + 1];
     b->widest_leaf = h[depth + 2];
     b->packed_stack = b->widest_leaf < 64 && b->nodes_used <= kPackMask + 1u && b->n_tris <= kPackMask + 1u;
+    if (!b->packed_stack) {
+        blas_buffer_release(ctx, b->d_wide, wide_bytes(b->node_count));
+        b->d_wide = nullptr;
+    }
     (void)hipFree(b->d_big_leaves);
     b->d_big_leaves = nullptr;
     b->n_big_leaves = nbig;
@@ -1392,7 +1446,7 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
         if (rc)
             return rc;
         hipLaunchKernelGGL(k_big_leaves, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, big,
-                           b->d_big_leaves, nullptr, 0u);
+                           b->d_big_leaves, nullptr, 0u, nullptr, nullptr);
         BVHT_HIP(hipGetLastError());
     }
     BVHT_HIP(hipStreamSynchronize(st));
@@ -1409,7 +1463,7 @@ int32_t launch_refit(bvht_ctx ctx, bvht_blas blas)
         hipLaunchKernelGGL(k_refit_big_leaves, dim3(blocks_for(blas->n_big_leaves, 4)), dim3(256), 0, ctx->stream,
                            blas->d_nodes, blas->d_tris, blas->d_big_leaves, blas->n_big_leaves);
     hipLaunchKernelGGL(k_refit_chunks, dim3(chunk_count(blas->nodes_used)), dim3(kChunkWG), 0, ctx->stream,
-                       blas->d_nodes, blas->d_tris, blas->d_level, blas->d_chunks);
+                       blas->d_nodes, blas->d_tris, blas->d_level, blas->d_chunks, blas->d_wide);
     LevelRun run{};
     auto flush = [&]() {
         if (run.levels)
@@ -1433,6 +1487,7 @@ int32_t launch_refit(bvht_ctx ctx, bvht_blas blas)
             flush();
     }
     flush();
+    launch_wide(ctx, blas);
     BVHT_HIP(hipGetLastError());
     return BVHT_OK;
 }
@@ -1581,6 +1636,27 @@ static int leaf_group(bvht_blas b, uint32_t n)
     return mean >= 64 ? 8 : 0;
 }
 
+// Four lanes a ray where the launch is as long as its longest rays: a quad's
+// step is shorter and there are half as many, but four times the waves share
+// the vector units.  Camera rays (us, a lane a ray / quads with 1, 8 and 16
+// rays a wave), soup of 12,582 triangles and sphere of 20,480:
+//   64 rays         58 / 37 /  42 /  42     39 / 20 / 28 / 29
+//   4,096          111 / 66 /  91 /  96     46 / 35 / 31 / 32
+//   16,384         114 / 80 /  96 /  91     53 / 63 / 38 / 37
+//   65,536         135 / 107 / 105 / 110    58 / 155 / 57 / 46
+//   160,000        158 / 167 / 114 / 117    58 / 323 / 78 / 64
+// and the same order on random rays (64 rays 88 / 51 and 36 / 22, 65,536 298 /
+// 204 and 81 / 61, 200,000 278 / 304 and 90 / 103 with 1 and 16).
+uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n)
+{
+    // (the autotuner's configurations, the wave order and a stack limit below
+    // the tree's bound are the lane-a-ray kernel's)
+    if (!blas->d_wide || n > 65536 || ctx->trace_wg > 0 || ctx->tls_on ||
+        (ctx->stack_limit && ctx->stack_limit + 1 < blas->depth))
+        return 0;
+    return n <= 4096 ? 1 : (n <= 16384 ? 8 : 16);
+}
+
 int32_t launch_trace_blas(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_rays, uint32_t n,
                           const uint32_t* d_n, bvht_hit* d_hits, bvht_stats* d_stats)
 {
@@ -1593,8 +1669,11 @@ int32_t launch_trace_blas(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_rays, 
     // (a stack limit below the tree's bound limits the lane-a-ray kernel's stack)
     const bool capped = ctx->stack_limit && ctx->stack_limit + 1 < blas->depth;
     const int group = capped || d_stats || ctx->trace_wg > 0 || ctx->tls_on ? 0 : leaf_group(blas, n);
+    const uint32_t per = d_stats || group ? 0 : quad_rays(ctx, blas, n);
     if (group)
         lds = kGroupStack;
+    if (per)
+        lds = kQuadStack;
     uint32_t* spill = nullptr;
     if (need > (uint32_t)lds) {
         int32_t rc = ensure_spill(ctx, &ctx->spill, &ctx->spill_words, (size_t)(need - lds) * n);
@@ -1606,6 +1685,13 @@ int32_t launch_trace_blas(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_rays, 
         hipLaunchKernelGGL(group == 16 ? k_trace_group<16> : k_trace_group<8>, dim3(blocks_for(n, 256 / group)),
                            dim3(256), 0, ctx->stream, reinterpret_cast<const float4*>(blas->d_nodes), blas->d_tris,
                            d_rays, d_hits, n, d_n, spill, need, ctx->d_status);
+        BVHT_HIP(hipGetLastError());
+        return BVHT_OK;
+    }
+    if (per) {
+        hipLaunchKernelGGL(k_trace_quad, dim3(blocks_for(n, per)), dim3(64), 0, ctx->stream,
+                           reinterpret_cast<const float4*>(blas->d_nodes), blas->d_wide, blas->d_tris, d_rays, d_hits,
+                           n, d_n, spill, need, ctx->d_status, per);
         BVHT_HIP(hipGetLastError());
         return BVHT_OK;
     }
@@ -1996,6 +2082,8 @@ int32_t bvht_blas_upload(bvht_ctx ctx, const bvht_node* nodes, uint32_t node_cou
         return rc;
     b->nodes_used = nodes_used;
     b->one_parent = one_parent_each(nodes, nodes_used);
+    for (uint32_t k = 0; k < nodes_used; ++k)
+        b->even_pairs = b->even_pairs && (k == 1 || nodes[k].count > 0 || (nodes[k].left_first & 1u) == 0);
     rc = host_to_device(ctx, b->d_nodes, nodes, sizeof(bvht_node) * (size_t)node_count);
     if (!rc)
         rc = host_to_device(ctx, b->d_tris, tris, sizeof(float) * 9 * (size_t)n);
@@ -2090,6 +2178,7 @@ int32_t bvht_blas_destroy(bvht_blas b)
     blas_buffer_release(c, b->d_parent, sizeof(uint32_t) * nc);
     blas_buffer_release(c, b->d_level, sizeof(uint32_t) * nc);
     blas_buffer_release(c, b->d_level_order, sizeof(uint32_t) * nc);
+    blas_buffer_release(c, b->d_wide, wide_bytes(nc));
     blas_buffer_release(c, b->d_chunks, sizeof(uint32_t) * (chunk_count((uint32_t)nc) + 1));
     (void)hipFree(b->d_big_leaves);
     (void)hipFree(b->d_attr_normals);

@@ -275,6 +275,7 @@ __device__ __forceinline__ uint32_t dpp_u(uint32_t v)
 {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
 }
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E;  // quad_perm: lane ^ 1, lane ^ 2
 // The value of lane `lane ^ J` (J a power of two below 64) without LDS:
 // quad permutes for 1 and 2, row shifts for 4, a row rotate for 8, and the
 // permlane swaps (v_permlane16/32_swap: odd rows of the first operand with

@@ -303,6 +303,33 @@ __global__ __launch_bounds__(WG) void k_trace_forward(const float4* __restrict__
     }
 }
 
+// The forward with four lanes a ray (traverse_quad), `per` rays (1 to 16) a
+// wave.
+__global__ __launch_bounds__(64) void k_trace_forward_quad(const float4* __restrict__ nodes,
+                                                           const float4* __restrict__ wide,
+                                                           const float* __restrict__ tris,
+                                                           const uint32_t* __restrict__ vid,
+                                                           const float* __restrict__ normals, Rows rows, V3 light,
+                                                           const bvht_ray* __restrict__ rays, uint32_t n,
+                                                           bvht_hit* __restrict__ hits, float2* __restrict__ image,
+                                                           uint32_t* __restrict__ spill, uint32_t cap,
+                                                           uint32_t* __restrict__ status, uint32_t per)
+{
+    __shared__ uint32_t lds[kQuadLds * 64];
+    const uint32_t i = blockIdx.x * per + (threadIdx.x >> 2);
+    if ((threadIdx.x >> 2) >= per || i >= n)
+        return;
+    const float4* rp = reinterpret_cast<const float4*>(rays + i);
+    const float4 a = rp[0], b = rp[1];
+    const V3 o = rows_mul(rows.r0, rows.r1, rows.r2, mk3(a.x, a.y, a.z), 1.0f);
+    const V3 d = rows_mul(rows.r0, rows.r1, rows.r2, mk3(b.x, b.y, b.z), 0.0f);
+    const BlasResult r = trace_quad(nodes, wide, tris, make_ray(o, d, a.w), lds, spill + i, (size_t)n, cap, status);
+    if ((threadIdx.x & 3u) != 0)
+        return;
+    store_hit(hits, i, r.found, r.t, r.u, r.v, r.prim, 0);
+    image[i] = r.found ? make_float2(r.t, shade_at(normals, vid, r.prim, r.u, r.v, light)) : make_float2(kFltMax, 0.0f);
+}
+
 constexpr uint32_t kSchedGroups = 4096;
 
 typedef void (*forward_fn)(const float4*, const float*, const uint32_t*, const float*, Rows, V3, const bvht_ray*,
@@ -966,12 +993,23 @@ extern "C" int32_t bvht_trace_forward(bvht_ctx ctx, bvht_mesh mesh, const float*
     uint32_t need = stack_cap(ctx, b->depth > 0 ? b->depth - 1 : 0);
     int wg, lds;
     trace_config(ctx, need, &wg, &lds);
+    const uint32_t per = quad_rays(ctx, b, n);
+    if (per)
+        lds = kQuadStack;
     uint32_t* spill = nullptr;
     if (need > (uint32_t)lds) {
         int32_t rc = ensure_spill(ctx, &ctx->spill, &ctx->spill_words, (size_t)(need - lds) * n);
         if (rc)
             return rc;
         spill = ctx->spill;
+    }
+    if (per) {
+        hipLaunchKernelGGL(k_trace_forward_quad, dim3(nblk(n, per)), dim3(64), 0, ctx->stream,
+                           reinterpret_cast<const float4*>(b->d_nodes), b->d_wide, b->d_tris, mesh->d_vid,
+                           mesh->d_normals, rows_of(minv), V3{light[0], light[1], light[2]}, d_rays, n, d_hits,
+                           reinterpret_cast<float2*>(d_image), spill, need, ctx->d_status, per);
+        BVHT_HIP(hipGetLastError());
+        return BVHT_OK;
     }
     forward_fn fn = pick_forward(wg, lds, mesh->blas->packed_stack);
     if (!fn)

@@ -112,6 +112,7 @@ struct bvht_blas_s {
     bvht_node* d_nodes = nullptr;
     float* d_tris = nullptr;  // 9 floats per triangle, build order
     uint32_t* d_perm = nullptr;  // input index of the triangle at each build position (GPU builds only)
+    float4* d_wide = nullptr;           // wide records (bvht_trace.hpp), small packed trees only; NULL: none
     uint32_t* d_parent = nullptr;       // parent of each used node of an uploaded tree (root: 0xFFFFFFFF)
     uint32_t* d_level = nullptr;        // depth of each used node (root 0; dummy node 1: 0xFFFFFFFF), bit 31: refit_chunk's
     uint32_t* d_level_order = nullptr;  // the nodes refit_chunk leaves, grouped by level
@@ -120,6 +121,7 @@ struct bvht_blas_s {
     uint32_t* d_big_leaves = nullptr;   // leaves with more than kBigLeaf triangles (refit a wave each)
     uint32_t n_big_leaves = 0;
     bool one_parent = true;     // no node has two parents (an uploaded tree's may)
+    bool even_pairs = true;     // child pairs at even indices (an uploaded tree's may not be)
     uint32_t widest_leaf = 0;   // triangles of the largest leaf (0 if below 64 and leaves are small on average)
     bool packed_stack = false;  // every node fits a packed stack entry (see bvht_trace.hpp)
     // shading attributes (bvht_blas_set_attributes)
@@ -192,6 +194,9 @@ inline uint32_t stack_cap(bvht_ctx ctx, uint32_t need)
 {
     return (ctx->stack_limit && ctx->stack_limit < need) ? ctx->stack_limit : need;
 }
+// Rays a wave for a trace of n rays over blas with four lanes a ray, 0 for a
+// lane a ray.
+uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n);
 int32_t blas_alloc(bvht_ctx ctx, uint32_t n, uint32_t node_count, bvht_blas* out);
 // Frees the context's BLAS build workspace (bvht_destroy).
 void release_build_ws(bvht_ctx ctx);

@@ -8,6 +8,9 @@ namespace bvht {
 // LDS (address space 3) pointer, so stack accesses compile to ds_read/ds_write
 // instead of flat accesses.
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
+// 64-bit words of the same memory (may_alias: the two views of a wave's LDS
+// follow one another, and their accesses must not be reordered)
+typedef __attribute__((address_space(3), may_alias)) uint64_t lds_u64;
 
 // 64 bytes at a wave-uniform, 4-byte aligned address, loaded once for the
 // wave through the scalar data cache into 16 SGPRs.  The wait is inside the
@@ -296,6 +299,280 @@ __device__ __forceinline__ BlasResult traverse_group(const float4* __restrict__ 
     if (prim != BVHT_MISS && closest < kFltMax)
         res.found = tri_test(tris + 9 * (size_t)prim, ray, res.t, res.u, res.v);
     return res;
+}
+
+// ------------------------------------------------------ wide records --
+// Two binary levels in one fetch.  For every interior node x at even depth
+// the record at wide + 4 * left_first(x) (128 bytes, one L2 line) holds x's up
+// to four grandchildren, slots 0 and 1 below the left child and 2 and 3 below
+// the right, each {lo.xyz, ref}{hi.xyz, 0} (packed trees only).  A leaf's ref
+// is a packed stack entry (kPackFlag | count << kPackShift | left_first), an
+// interior node's its left_first.  A child that is a leaf fills its first
+// slot; the second has ref kNoRef and a box of NaNs, which nothing hits and
+// minima and maxima pass over.  Record 0 belongs to no node (left_first >= 2);
+// its first word is 1 when some node breaks what traverse_quad relies on.
+constexpr uint32_t kNoRef = 0xFFFFFFFFu;
+constexpr uint32_t kPairRef = 1u << 26;  // side (bit 25) of the record in bits 0..24
+
+__device__ __forceinline__ bool same_box(float4 lo, float4 hi, float4 alo, float4 ahi, float4 blo, float4 bhi)
+{
+    return lo.x == fminf(alo.x, blo.x) && lo.y == fminf(alo.y, blo.y) && lo.z == fminf(alo.z, blo.z) &&
+           hi.x == fmaxf(ahi.x, bhi.x) && hi.y == fmaxf(ahi.y, bhi.y) && hi.z == fmaxf(ahi.z, bhi.z);
+}
+__device__ __forceinline__ bool ordered_box(float4 lo, float4 hi)
+{
+    return lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z;
+}
+
+// Writes node k's wide record (nothing for a leaf).  Marks the tree when the
+// node's box is not the union of its children's, a child's not the union of
+// the grandchildren's, or a box has lo > hi or a NaN (uploaded trees, NaN
+// vertices): called for every node at even depth it looks at every box.
+__device__ __forceinline__ void write_wide(const float4* __restrict__ nodes, float4* __restrict__ wide, uint32_t k)
+{
+    const float4 xlo = nodes[2 * (size_t)k], xhi = nodes[2 * (size_t)k + 1];
+    if (__float_as_uint(xhi.w) != 0)
+        return;
+    const uint32_t lf = __float_as_uint(xlo.w);
+    const float4* c = nodes + 2 * (size_t)lf;
+    float4 lo[4], hi[4];
+    uint32_t ref[4];
+    const float4 clo[2] = {c[0], c[2]}, chi[2] = {c[1], c[3]};
+    bool ok = same_box(xlo, xhi, clo[0], chi[0], clo[1], chi[1]);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const uint32_t cnt = __float_as_uint(chi[s].w), clf = __float_as_uint(clo[s].w);
+        if (cnt) {
+            const float nan = __uint_as_float(0x7FC00000u);
+            lo[2 * s] = clo[s];
+            hi[2 * s] = chi[s];
+            lo[2 * s + 1] = hi[2 * s + 1] = make_float4(nan, nan, nan, nan);
+            ref[2 * s] = kPackFlag | cnt << kPackShift | clf;
+            ref[2 * s + 1] = kNoRef;
+        } else {
+            const float4* g = nodes + 2 * (size_t)clf;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                lo[2 * s + j] = g[2 * j];
+                hi[2 * s + j] = g[2 * j + 1];
+                const uint32_t n = __float_as_uint(hi[2 * s + j].w), f = __float_as_uint(lo[2 * s + j].w);
+                ref[2 * s + j] = n ? kPackFlag | n << kPackShift | f : f;
+            }
+            ok = ok && same_box(clo[s], chi[s], lo[2 * s], hi[2 * s], lo[2 * s + 1], hi[2 * s + 1]);
+        }
+        ok = ok && ordered_box(lo[2 * s], hi[2 * s]) && (cnt || ordered_box(lo[2 * s + 1], hi[2 * s + 1]));
+    }
+    float4* w = wide + 4 * (size_t)lf;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        w[2 * k] = make_float4(lo[k].x, lo[k].y, lo[k].z, __uint_as_float(ref[k]));
+        w[2 * k + 1] = make_float4(hi[k].x, hi[k].y, hi[k].z, 0.0f);
+    }
+    if (!ok)
+        *reinterpret_cast<uint32_t*>(wide) = 1u;
+}
+
+// Whether the wide records may trace this ray: t not above FLT_MAX, a finite
+// origin, and no reciprocal direction that is 0 or NaN (an infinite one, from
+// a zero direction component, is allowed).
+__device__ __forceinline__ bool wide_ray(const DRay& r)
+{
+    return !(r.t > kFltMax) && fabsf(r.o.x) <= kFltMax && fabsf(r.o.y) <= kFltMax && fabsf(r.o.z) <= kFltMax &&
+           fabsf(r.r.x) > 0.0f && fabsf(r.r.y) > 0.0f && fabsf(r.r.z) > 0.0f;
+}
+__device__ __forceinline__ bool finite_dir(const DRay& r)
+{
+    return fabsf(r.r.x) <= kFltMax && fabsf(r.r.y) <= kFltMax && fabsf(r.r.z) <= kFltMax;
+}
+
+// traverse_blas with four lanes a ray on the wide records: lane q of a quad
+// holds slot q, so a step is one slab test instead of four, and a leaf's
+// triangles are tested four at a time.  The same leaves are tested in the same
+// order with the same nearest hit, in about half the steps.  Why the hits are
+// the same bit for bit:
+// - binary32 subtraction and multiplication are monotone and each child's
+//   box is the union of its children's, so a child's distance on an axis is
+//   the smaller of the grandchildren's, its key is the maximum of those over
+//   the axes, and a grandchild is hit only if the child is.  So the child
+//   order follows from the grandchildren's boxes, and a child whose
+//   grandchildren all miss is entered in vain.
+// - An infinite reciprocal and a bound equal to the origin give 0 * inf =
+//   NaN, which breaks this: with such a ray in the wave (`degen`) the
+//   children's boxes are tested too.
+// - The near side's grandchildren are tested now, as in the binary loop.  The
+//   far side's are tested in the binary loop when the far child is popped,
+//   against the distance found by then: the far side is pushed as a pair
+//   (the record and the side) and its half of the record tested at the pop.
+// - Each entry has its key and is dropped at the pop when that is not below
+//   the nearest hit: every test below it would fail.  A leaf already decided
+//   on has key -inf.
+// - A leaf's triangles are taken by distance, then by index: the sequential
+//   loop's first nearest one.
+// All four lanes of a quad hold the same ray and state.  st: this quad's
+// column of kQuadSlots {ref, key} entries, 16 apart; a ray that
+// needs more stops with `overflow`.
+// The child order is worked out on lane masks (a bit a lane, in scalar
+// registers): a step's logic then costs the vector units nothing.
+constexpr uint32_t kQuadLds = 16;                 // LDS words a lane
+constexpr uint32_t kQuadSlots = 2 * kQuadLds;     // entries a ray
+constexpr int kQuadStack = 4 * (int)kQuadLds;     // LDS stack entries a ray of the binary loop
+
+constexpr uint64_t kEven = 0x5555555555555555ull, kLow2 = 0x3333333333333333ull;  // lanes q & 1 == 0, q < 2
+__device__ __forceinline__ uint64_t lanes_of(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+__device__ __forceinline__ bool lane_in(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+__device__ __forceinline__ uint64_t mask_xor1(uint64_t m) { return (m & kEven) << 1 | (m >> 1 & kEven); }
+__device__ __forceinline__ uint64_t mask_xor2(uint64_t m) { return (m & kLow2) << 2 | (m >> 2 & kLow2); }
+// min(a, b) of operands that are never signalling NaNs: no canonicalizes
+__device__ __forceinline__ float min_raw(float a, float b)
+{
+    return __builtin_amdgcn_fmed3f(a, b, __uint_as_float(0xFF800000u));
+}
+
+__device__ __forceinline__ BlasResult traverse_quad(const float4* __restrict__ nodes, const float4* __restrict__ wide,
+                                                    const float* __restrict__ tris, const DRay& ray, bool degen,
+                                                    lds_u64* st, bool& overflow)
+{
+    constexpr uint32_t kPop = 0xFFFFFFFEu, kDone = 0xFFFFFFFDu, kFull = 0xFFFFFFFCu;  // no leaf's ref (packed_stack)
+    const uint32_t q = threadIdx.x & 3u;
+    const uint32_t pair_bits = kPairRef | (q >> 1) << kPackShift;
+    const float neg_inf = __uint_as_float(0xFF800000u);
+    float closest = ray.t;
+    uint32_t prim = BVHT_MISS, sp = 0;
+    const uint32_t root = __float_as_uint(nodes[0].w), root_cnt = __float_as_uint(nodes[1].w);
+    // current node: an interior node or a pair below kPackFlag, a leaf below
+    // kFull, kFull (out of entries), kDone, kPop
+    uint32_t cur = root_cnt ? kPackFlag | root_cnt << kPackShift | root : root;
+    while (true) {
+        while ((int32_t)cur >= 0) {
+            const uint32_t rec = cur & kPackMask;
+            const float4* at = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(wide) +
+                                                               ((rec << 6) + (q << 5)));
+            const float4 lo = at[0], hi = at[1];
+            const uint32_t ref = __float_as_uint(lo.w);
+            const float x1 = (lo.x - ray.o.x) * ray.r.x, x2 = (hi.x - ray.o.x) * ray.r.x;
+            const float y1 = (lo.y - ray.o.y) * ray.r.y, y2 = (hi.y - ray.o.y) * ray.r.y;
+            const float z1 = (lo.z - ray.o.z) * ray.r.z, z2 = (hi.z - ray.o.z) * ray.r.z;
+            const float nx = fminf(x1, x2), ny = fminf(y1, y2), nz = fminf(z1, z2);
+            const float tmin = fmaxf(fmaxf(nx, ny), nz);
+            const float tmax = fminf(fminf(fmaxf(x1, x2), fmaxf(y1, y2)), fmaxf(z1, z2));
+            // a pair's step takes its side only: in the lanes of the other side
+            // its two bits differ from theirs in the side
+            const uint64_t out = lanes_of(((cur >> kPackShift) ^ (pair_bits >> kPackShift)) == 1u);
+            uint64_t hit = lanes_of(tmax >= tmin) & lanes_of(tmax > 0.0f) & ~out;
+            // the child's key (meant only where it is hit)
+            float kp = fmaxf(fmaxf(min_raw(nx, dpp_f<kXor1>(nx)), min_raw(ny, dpp_f<kXor1>(ny))),
+                             min_raw(nz, dpp_f<kXor1>(nz)));
+            if (degen) {
+                kp = slab_key(make_float4(fminf(lo.x, dpp_f<kXor1>(lo.x)), fminf(lo.y, dpp_f<kXor1>(lo.y)),
+                                          fminf(lo.z, dpp_f<kXor1>(lo.z)), 0.0f),
+                              make_float4(fmaxf(hi.x, dpp_f<kXor1>(hi.x)), fmaxf(hi.y, dpp_f<kXor1>(hi.y)),
+                                          fmaxf(hi.z, dpp_f<kXor1>(hi.z)), 0.0f),
+                              ray);
+                hit &= lanes_of(kp < closest) | lanes_of((cur & kPairRef) != 0);
+            }
+            const float key = lane_in(hit) ? tmin : kFltMax;
+            // the side's nearer grandchild first, ties to the right one; then
+            // the nearer side, ties to the right one
+            const float kn = dpp_f<kXor1>(key), kpo = dpp_f<kXor2>(kp);
+            const uint64_t first = (lanes_of(key < kn) & kEven) | (lanes_of(key <= kn) & ~kEven);
+            const uint64_t below = lanes_of(key < closest);
+            const uint64_t pass = below | mask_xor1(below), pass_o = mask_xor2(pass);
+            const uint64_t near =
+                pass & (~pass_o | (lanes_of(kp < kpo) & kLow2) | (lanes_of(kp <= kpo) & ~kLow2));
+            const uint64_t both = pass & pass_o;
+            const uint32_t rn = dpp_u<kXor1>(ref);
+            const uint32_t ra = lane_in(first) ? ref : rn;
+            const float ks = lane_in(first) ? kn : key;
+            const uint32_t rao = dpp_u<kXor2>(ra);
+            const float kso = dpp_f<kXor2>(ks);
+            // the near side's second grandchild, and the far side: a leaf
+            // child, or the pair
+            const uint64_t second = lanes_of((lane_in(near) ? ks : kso) < closest) & (pass | pass_o);
+            const uint64_t push = (below & near & ~first) | (both & first & ~near);
+            if (lane_in(push)) {
+                const uint64_t child = lanes_of(rn == kNoRef) & ~near;  // far leaf children
+                const uint64_t leaf = lanes_of((int32_t)ref < 0);
+                const uint32_t e = lane_in(near | child) ? ref : rec | pair_bits;
+                const uint32_t k = __float_as_uint(lane_in((near & leaf) | child) ? neg_inf : key);
+                st[(sp + (lane_in(near & both) ? 1u : 0u)) * 16] = (uint64_t)k << 32 | e;
+            }
+            sp += (lane_in(both) ? 1u : 0u) + (lane_in(second) ? 1u : 0u);
+            const uint32_t next = lane_in(near) ? ra : rao;
+            cur = sp > kQuadSlots - 2 ? kFull : lane_in(pass | pass_o) ? next : kPop;
+            if ((uint32_t)__popcll(lanes_of((int32_t)cur >= 0)) < kDescendMin)
+                break;
+        }
+        if ((int32_t)cur < 0 && cur < kFull) {
+            const uint32_t begin = cur & kPackMask, cnt = (cur >> kPackShift) & 63u;
+            float bt = closest;
+            uint32_t bi = BVHT_MISS;
+            for (uint32_t k = q; k < cnt; k += 4) {
+                float t, u, v;
+                if (tri_test(tris + 9 * (size_t)(begin + k), ray, t, u, v) && t < bt) {
+                    bt = t;
+                    bi = begin + k;
+                }
+            }
+            float ot = dpp_f<kXor1>(bt);
+            uint32_t oi = dpp_u<kXor1>(bi);
+            bool take = lane_in(lanes_of(ot < bt) | (lanes_of(ot == bt) & lanes_of(oi < bi)));
+            bt = take ? ot : bt;
+            bi = take ? oi : bi;
+            ot = dpp_f<kXor2>(bt);
+            oi = dpp_u<kXor2>(bi);
+            take = lane_in(lanes_of(ot < bt) | (lanes_of(ot == bt) & lanes_of(oi < bi)));
+            closest = take ? ot : bt;
+            bi = take ? oi : bi;
+            prim = bi != BVHT_MISS ? bi : prim;
+            cur = kPop;
+        }
+        if (cur == kPop) {
+            cur = kDone;
+            while (sp > 0) {
+                --sp;
+                const uint64_t e = st[sp * 16];
+                if (__uint_as_float((uint32_t)(e >> 32)) < closest) {
+                    cur = (uint32_t)e;
+                    break;
+                }
+            }
+        }
+        if (cur == kDone || cur == kFull)
+            break;
+        __builtin_amdgcn_wave_barrier();  // one loop latch for every lane (see traverse_blas)
+    }
+    overflow = cur == kFull;
+    // the hit's t, u and v again from its triangle: the same arithmetic
+    BlasResult res{0.0f, 0.0f, 0.0f, prim, false};
+    if (prim != BVHT_MISS && closest < kFltMax)
+        res.found = tri_test(tris + 9 * (size_t)prim, ray, res.t, res.u, res.v);
+    return res;
+}
+
+// One ray of a quad: traverse_quad where the tree's records are unmarked and
+// every ray of the wave allows it, else (and for a ray whose stack overflowed)
+// the binary loop in the quad's first lane, with the quad's LDS as its stack.
+// The result is the first lane's.  lds: kQuadLds words for each lane of the
+// workgroup; each wave keeps to its own.
+__device__ __forceinline__ BlasResult trace_quad(const float4* __restrict__ nodes, const float4* __restrict__ wide,
+                                                 const float* __restrict__ tris, const DRay& ray, uint32_t* lds,
+                                                 uint32_t* spill, size_t stride, uint32_t cap, uint32_t* status)
+{
+    lds_u32* wave = (lds_u32*)(lds + (threadIdx.x >> 6) * (64 * kQuadLds));
+    const uint32_t lane = threadIdx.x & 63u;
+    BlasResult r{0.0f, 0.0f, 0.0f, 0u, false};
+    bool again = true;
+    if (*reinterpret_cast<const uint32_t*>(wide) == 0 && __builtin_amdgcn_ballot_w64(!wide_ray(ray)) == 0)
+        r = traverse_quad(nodes, wide, tris, ray, __builtin_amdgcn_ballot_w64(!finite_dir(ray)) != 0,
+                          reinterpret_cast<lds_u64*>(wave) + (lane >> 2), again);
+    // (the ballot keeps the binary loop behind the other for the whole wave:
+    // both use its LDS)
+    if (__builtin_amdgcn_ballot_w64(again) != 0 && again && (lane & 3u) == 0) {
+        Stack<kQuadStack, 16> st{wave + (lane >> 2), spill, stride, cap, status};
+        uint32_t pairs = 0, tests = 0;
+        r = traverse_blas<false, true, false>(nodes, tris, ray, st, 0u, pairs, tests);
+    }
+    return r;
 }
 
 // Per-BLAS device pointers used by the TLAS kernels.

@@ -182,8 +182,11 @@ __device__ __forceinline__ void mark_chunk(const bvht_node* __restrict__ nodes, 
 }
 
 __device__ __forceinline__ void refit_chunk(bvht_node* __restrict__ nodes, const float* __restrict__ tris,
-                                            const uint32_t* __restrict__ level, uint32_t base, uint32_t end)
+                                            const uint32_t* __restrict__ level, uint32_t base, uint32_t end,
+                                            float4* __restrict__ wide)
 {
+    if (wide && base == 0 && threadIdx.x == 0)
+        *reinterpret_cast<uint32_t*>(wide) = 0;  // the mark, set again by the records' writing
     __shared__ float box[6][kRefitChunk];
     uint32_t lv[kChunkPer], lf[kChunkPer];
     for (uint32_t j = 0; j < kChunkPer; ++j) {

@@ -546,3 +546,68 @@ def test_trees_with_large_leaves(ctx, orc, mesh, n):
     assert_hits_equal(bvh.intersect(rays), ref, f"{mesh} {n}")
     assert n < 100 or (ref["prim"] != B.MISS).sum() > 5
     bvh.close()
+
+
+def flat_grid(k):
+    """k x k unit cells of two triangles each in the plane z = 0: flat boxes
+    with bounds at whole numbers."""
+    x, y = [a.ravel().astype(np.float32) for a in np.meshgrid(np.arange(k), np.arange(k), indexing="ij")]
+    z = np.zeros_like(x)
+    a, b, c, d = [np.stack(p, 1) for p in ((x, y, z), (x + 1, y, z), (x, y + 1, z), (x + 1, y + 1, z))]
+    return np.ascontiguousarray(np.concatenate([np.concatenate([a, b, c], 1), np.concatenate([b, d, c], 1)]))
+
+
+@pytest.mark.parametrize("tree,n", [("soup", 1), ("soup", 15), ("soup", 4096), ("soup", 4097), ("soup", 16385),
+                                    ("soup", 65536), ("soup", 65537), ("two", 500), ("grid", 9000), ("comb", 3000),
+                                    ("loose", 3000), ("odd", 3000), ("nan", 3000)])
+def test_small_launches_over_small_trees(ctx, orc, tree, n):
+    """Up to 65,536 rays over a small tree take four lanes a ray on the wide
+    records; hits are the oracle's bit for bit, also after a refit.  Rays per
+    wave 1, 8 and 16; zero direction components, with origins on box bounds
+    (0 * inf in the slab test) over flat boxes; t = +inf and NaN; a comb of
+    150 levels that outgrows the entries; trees that the records do not fit:
+    boxes larger than their children's union, child pairs at odd indices, NaN
+    vertices from a refit."""
+    if tree == "comb":
+        nodes, used, tris = comb_tree(150)
+    else:
+        mesh = flat_grid(24) if tree == "grid" else scenes.triangle_soup(2 if tree == "two" else 3000, seed=41)
+        nodes, used, tris = orc.bvh_build(mesh, False, 2)
+    if tree == "loose":
+        nodes["bmin"][2:used:3] -= np.float32(0.25)
+    if tree == "odd":
+        moved = np.zeros(used + 1, B.NODE_DTYPE)
+        moved[0], moved[3:] = nodes[0], nodes[2:used]
+        moved["left_first"] += (moved["count"] == 0).astype(np.uint32)
+        moved["left_first"][1:3], moved["count"][1:3] = 0, 1
+        nodes, used = moved, used + 1
+    bvh = upload(ctx, nodes, used, tris)
+    rays = random_rays(n, 99)
+    if tree == "grid":
+        rays["o"] = np.round(rays["o"] * 2.0) + np.float32(12.0)
+        rays["o"][::5, 2] = 0.0
+    elif tree == "two":
+        rays["d"] = tris.reshape(-1, 3, 3).mean(1)[np.arange(n) % 2] + np.float32(0.2) * rays["d"] - rays["o"]
+    elif tree == "comb":
+        rays["o"] = rays["o"] * np.float32([0.0, 0.1, 0.1]) + np.float32([-5.0, 0.0, 0.0])
+        rays["d"] = (1.0, 1e-3, -1e-3)
+    rays["d"][5::7, 0] = 0.0
+    rays["d"][6::9, 1] = -0.0
+    rays["d"][8::11, :2] = 0.0
+    rays["tmax"][3::70] = np.inf
+    rays["tmax"][10::310] = np.nan
+    rays["o"][20::500] = np.inf
+    want = nodes.copy()
+    for step in range(2):
+        ref = orc.bvh_trace(want, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+        assert_hits_equal(bvh.intersect(rays), ref, f"{tree} {n} {step}")
+        assert n < 100 or (ref["prim"] != B.MISS).sum() > 5
+        tris = tris.copy()
+        if tree == "nan":
+            tris[7::50, 0] = np.nan
+            tris[8::50] = np.nan
+        else:
+            tris[:, 1::3] += np.float32(0.125) * tris[:, 0::3]
+        bvh.refit(tris)
+        orc.bvh_refit(want, used, tris)
+    bvh.close()
