@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "bvht_device.hpp"
@@ -75,10 +76,14 @@ struct Decision {
 };
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
-// Per split node, the keys part_commit_chunk reduces for its two children:
+// Per split node, the keys part_scatter_chunk reduces for its two children:
 // mins (box lo left, right; centroid min left, right) then maxes (box hi
 // left, right; centroid max left, right), three each.
 constexpr uint32_t kChildKeys = 24;
+
+// Marks a small root (an entry of small_roots) whose elements are in the
+// second element buffer; node indices stay below 2 * 2^30.
+constexpr uint32_t kOther = 0x80000000u;
 
 // A node of the large-node tree: every node split level by level, their
 // children, and the small subtrees' roots.  Children are allocated in pairs
@@ -170,7 +175,7 @@ __device__ __forceinline__ void block_reduce_keys(uint32_t (&vals)[NV], uint32_t
 
 // Per triangle: centroid, vertex min/max, original index.
 __global__ void k_init_elems(const float* __restrict__ tris, uint32_t n, float4* __restrict__ ec,
-                             float4* __restrict__ elo, float2* __restrict__ ehi)
+                             float4* __restrict__ elo, float2* __restrict__ ehi, uint32_t* __restrict__ perm)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
@@ -183,6 +188,7 @@ __global__ void k_init_elems(const float* __restrict__ tris, uint32_t n, float4*
     ec[i] = make_float4(c.x, c.y, c.z, __uint_as_float(i));
     elo[i] = make_float4(lo.x, lo.y, lo.z, hi.x);
     ehi[i] = make_float2(hi.y, hi.z);
+    perm[i] = i;
 }
 
 // Accumulators of the level's L large nodes, by workgroup g of `groups`.  Run
@@ -594,6 +600,25 @@ __global__ void k_part_prefix(const uint32_t* __restrict__ node_chunk_begin, con
     }
 }
 
+// One element's box and centroid into the keys of side SIDE / 3 of its node.
+template <int SIDE>
+__device__ __forceinline__ void child_key_step(uint32_t (&v)[kChildKeys], const float4& c, const float4& lo,
+                                               const float2& hi)
+{
+    key_min(v[SIDE + 0], lo.x);
+    key_min(v[SIDE + 1], lo.y);
+    key_min(v[SIDE + 2], lo.z);
+    key_min(v[6 + SIDE + 0], c.x);
+    key_min(v[6 + SIDE + 1], c.y);
+    key_min(v[6 + SIDE + 2], c.z);
+    key_max(v[12 + SIDE + 0], lo.w);
+    key_max(v[12 + SIDE + 1], hi.x);
+    key_max(v[12 + SIDE + 2], hi.y);
+    key_max(v[18 + SIDE + 0], c.x);
+    key_max(v[18 + SIDE + 1], c.y);
+    key_max(v[18 + SIDE + 2], c.z);
+}
+
 // Two-pointer partition (bvh.rs:420-429) as a permutation.  With n elements
 // at relative positions k, nl of them "left" (centroid < split):
 //   the examined sequence takes the next left-stream element after a left-goer
@@ -607,13 +632,25 @@ __global__ void k_part_prefix(const uint32_t* __restrict__ node_chunk_begin, con
 //   Right-goers of the right stream move down by one.
 // Phase A records, per node, kpos[m] (position of the m-th left-stream
 // right-goer) and sel[m] (top-index of the m-th right-stream left-goer).
+// Phase B moves the elements into the other of the two element buffers, whose
+// part of the node's range nobody reads in this level, writes the positions
+// the final order needs (perm) and reduces what the split needs of them, by
+// the side they land on: the two child boxes (update_node_bounds of the
+// children, bvh.rs:462-463) and the children's centroid ranges (the next
+// level's find_best_split_plane, bvh.rs:338-344).
+// Bound by its scattered stores and, below some 100k elements, by the launch.
+// A third pass that copied the elements back and reduced them there read and
+// wrote another 80 bytes an element: 1.3M triangles 6,565 -> 6,305 us without
+// it, in reference mode 3,225 -> 3,135; 12.6k 836 -> 785, in reference mode
+// 806 -> 735 (one launch a level fewer).
 template <bool PHASE_B>
 __device__ void part_scatter_chunk(const float4* __restrict__ ec, const float4* __restrict__ elo,
                                    const float2* __restrict__ ehi, Chunk ch, uint32_t base,
                                    const Task* __restrict__ tasks, const Decision* __restrict__ dec,
                                    uint32_t* __restrict__ kpos, uint32_t* __restrict__ sel, float4* __restrict__ oc,
-                                   float4* __restrict__ olo, float2* __restrict__ ohi, uint32_t* __restrict__ err,
-                                   uint32_t* wc)
+                                   float4* __restrict__ olo, float2* __restrict__ ohi, uint32_t* __restrict__ perm,
+                                   uint32_t* __restrict__ child_keys, uint32_t* __restrict__ err, uint32_t* wc,
+                                   uint32_t* lds)
 {
     Decision d = dec[ch.slot];
     if (d.kind == 0)
@@ -627,6 +664,12 @@ __device__ void part_scatter_chunk(const float4* __restrict__ ec, const float4* 
         float v = d.axis == 0 ? c.x : (d.axis == 1 ? c.y : c.z);
         a = (v < d.pos) ? nl : nl + 1;
     }
+    // a plane split that leaves one side empty is abandoned (bvh.rs:431-435),
+    // or replaced by the median split when the node must be split
+    const uint32_t nleft = d.kind == 1 && nl != 0 && nl != n ? nl : n / 2;
+    uint32_t v[kChildKeys];
+    for (uint32_t q = 0; q < kChildKeys; ++q)
+        v[q] = q < kChildKeys / 2 ? kEmptyMin : kEmptyMax;
     for (uint32_t e0 = ch.begin; e0 < ch.end; e0 += kWG) {
         uint32_t e = e0 + threadIdx.x;
         bool in = e < ch.end;
@@ -653,14 +696,8 @@ __device__ void part_scatter_chunk(const float4* __restrict__ ec, const float4* 
         if (!in)
             continue;
         uint32_t k = e - first;
-        if (d.kind == 2) {
-            if (PHASE_B) {
-                oc[e] = c;
-                olo[e] = elo[e];
-                ohi[e] = ehi[e];
-            }
+        if (!PHASE_B && d.kind == 2)
             continue;
-        }
         // every index below is range-checked: a violation flags the build as
         // failed instead of touching memory outside the node's range
         if (!PHASE_B) {
@@ -680,7 +717,9 @@ __device__ void part_scatter_chunk(const float4* __restrict__ ec, const float4* 
             continue;
         }
         uint32_t dest = n;
-        if (k < a) {
+        if (d.kind == 2) {
+            dest = k;
+        } else if (k < a) {
             if (f) {
                 dest = k;
             } else {
@@ -709,7 +748,16 @@ __device__ void part_scatter_chunk(const float4* __restrict__ ec, const float4* 
         oc[first + dest] = c;
         olo[first + dest] = lo;
         ohi[first + dest] = hi;
+        if (d.kind == 1)
+            perm[first + dest] = __float_as_uint(c.w);
+        if (dest < nleft) {
+            child_key_step<0>(v, c, lo, hi);
+        } else {
+            child_key_step<3>(v, c, lo, hi);
+        }
     }
+    if (PHASE_B)
+        block_reduce_keys<kChildKeys>(v, child_keys + kChildKeys * (size_t)ch.slot, lds);
 }
 
 template <bool PHASE_B>
@@ -720,70 +768,15 @@ __global__ __launch_bounds__(kWG) void k_part_scatter(const float4* __restrict__
                                                       const uint32_t* __restrict__ chunk_left,
                                                       uint32_t* __restrict__ kpos, uint32_t* __restrict__ sel,
                                                       float4* __restrict__ oc, float4* __restrict__ olo,
-                                                      float2* __restrict__ ohi, uint32_t* __restrict__ err)
+                                                      float2* __restrict__ ohi, uint32_t* __restrict__ perm,
+                                                      uint32_t* __restrict__ child_keys, uint32_t* __restrict__ err)
 {
     __shared__ uint32_t wc[4];
+    __shared__ uint32_t lds[PHASE_B ? kChildKeys * 4 : 1];
     uint32_t C = ctl->C;
     for (uint32_t ci = blockIdx.x; ci < C; ci += gridDim.x)
         part_scatter_chunk<PHASE_B>(ec, elo, ehi, chunks[ci], chunk_left[ci], tasks, dec, kpos, sel, oc, olo, ohi,
-                                    err, wc);
-}
-
-__device__ void part_commit_chunk(const float4* __restrict__ oc, const float4* __restrict__ olo,
-                                  const float2* __restrict__ ohi, Chunk ch, Task t, Decision d,
-                                  float4* __restrict__ ec, float4* __restrict__ elo, float2* __restrict__ ehi,
-                                  uint32_t* __restrict__ child_keys, uint32_t* lds)
-{
-    uint32_t nl = d.kind == 1 ? d.nl : t.count / 2;
-    // a plane split that leaves one side empty is abandoned (bvh.rs:431-435),
-    // or replaced by the median split when the node must be split
-    if (d.kind == 1 && (nl == 0 || nl == t.count))
-        nl = t.count / 2;
-    uint32_t v[kChildKeys];
-    for (uint32_t k = 0; k < kChildKeys; ++k)
-        v[k] = k < kChildKeys / 2 ? kEmptyMin : kEmptyMax;
-    for (uint32_t e = ch.begin + threadIdx.x; e < ch.end; e += kWG) {
-        float4 c = oc[e];
-        float4 lo = olo[e];
-        float2 hi = ohi[e];
-        ec[e] = c;
-        elo[e] = lo;
-        ehi[e] = hi;
-        int side = (e - t.first) < nl ? 0 : 3;
-        key_min(v[side + 0], lo.x);
-        key_min(v[side + 1], lo.y);
-        key_min(v[side + 2], lo.z);
-        key_min(v[6 + side + 0], c.x);
-        key_min(v[6 + side + 1], c.y);
-        key_min(v[6 + side + 2], c.z);
-        key_max(v[12 + side + 0], lo.w);
-        key_max(v[12 + side + 1], hi.x);
-        key_max(v[12 + side + 2], hi.y);
-        key_max(v[18 + side + 0], c.x);
-        key_max(v[18 + side + 1], c.y);
-        key_max(v[18 + side + 2], c.z);
-    }
-    block_reduce_keys<kChildKeys>(v, child_keys + kChildKeys * ch.slot, lds);
-}
-
-// Copy the partitioned ranges back and reduce the two child boxes
-// (update_node_bounds of the children, bvh.rs:462-463) and the children's
-// centroid ranges (the next level's find_best_split_plane, bvh.rs:338-344).
-__global__ __launch_bounds__(kWG) void k_part_commit(const float4* __restrict__ oc, const float4* __restrict__ olo,
-                                                     const float2* __restrict__ ohi, const Chunk* __restrict__ chunks,
-                                                     const Ctl* __restrict__ ctl, const Task* __restrict__ tasks,
-                                                     const Decision* __restrict__ dec, float4* __restrict__ ec,
-                                                     float4* __restrict__ elo, float2* __restrict__ ehi,
-                                                     uint32_t* __restrict__ child_keys)
-{
-    __shared__ uint32_t lds[kChildKeys * 4];
-    uint32_t C = ctl->C;
-    for (uint32_t ci = blockIdx.x; ci < C; ci += gridDim.x) {
-        Chunk ch = chunks[ci];
-        Decision d = dec[ch.slot];
-        if (d.kind != 0)
-            part_commit_chunk(oc, olo, ohi, ch, tasks[ch.slot], d, ec, elo, ehi, child_keys, lds);
-    }
+                                    perm, child_keys, err, wc, lds);
 }
 
 struct SNode {  // same layout as bvht_node; internal nodes hold a local pair index
@@ -980,16 +973,23 @@ constexpr int kSmallWavesPerWG = 4;
 // 8 waves per SIMD (64 VGPRs, two dwords spilled) rather than the 7 its 67
 // VGPRs allow: 1.3M build 6.81 -> 6.71 ms, reference mode 3.45 -> 3.35 ms.
 __global__ __launch_bounds__(64 * kSmallWavesPerWG) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_small_wave(
-    float4* __restrict__ ec, const float4* __restrict__ elo, const float2* __restrict__ ehi,
-    const BNode* __restrict__ bn, const uint32_t* __restrict__ small_roots, uint32_t nroots,
-    SNode* __restrict__ snodes, uint32_t* __restrict__ pairs_out, int faithful, uint32_t max_leaf,
+    const float4* __restrict__ ec, const float4* __restrict__ elo, const float2* __restrict__ ehi,
+    const float4* __restrict__ oc, const float4* __restrict__ olo, const float2* __restrict__ ohi,
+    uint32_t* __restrict__ perm, const BNode* __restrict__ bn, const uint32_t* __restrict__ small_roots,
+    uint32_t nroots, SNode* __restrict__ snodes, uint32_t* __restrict__ pairs_out, int faithful, uint32_t max_leaf,
     uint32_t* __restrict__ err)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t r = blockIdx.x * kSmallWavesPerWG + (threadIdx.x >> 6);
     if (r >= nroots)
         return;  // wave-uniform; no workgroup barrier below
-    BNode rn = bn[small_roots[r]];
+    const uint32_t root = small_roots[r];
+    BNode rn = bn[root & ~kOther];
+    if (root & kOther) {
+        ec = oc;
+        elo = olo;
+        ehi = ohi;
+    }
     const uint32_t first = rn.first, count = rn.count;
     if (count == 0 || count > kSmall) {
         if (lane == 0)
@@ -1186,7 +1186,7 @@ __global__ __launch_bounds__(64 * kSmallWavesPerWG) __attribute__((amdgpu_waves_
         sp += 2;
     }
     if (lane < count)
-        ec[first + lane] = c;
+        perm[first + lane] = __float_as_uint(c.w);
     if (lane < 1 + 2 * npairs) {
         SNode o;
         o.bmin[0] = nb0; o.bmin[1] = nb1; o.bmin[2] = nb2;
@@ -1219,7 +1219,7 @@ __global__ __launch_bounds__(64) void k_small_emit(const SNode* __restrict__ sno
     uint32_t deepest = 0;  // deepest level + 1 of this lane's subtree
     if (r < nroots) {
         uint8_t* ld = ldep + threadIdx.x * 2 * kSmall;
-        const SNode* s = snodes + 2 * (size_t)bn[small_roots[r]].first;
+        const SNode* s = snodes + 2 * (size_t)bn[small_roots[r] & ~kOther].first;
         uint32_t np = pairs[r], rk = rank[r], lv0 = root_level[r];
         ld[0] = 0;
         for (uint32_t j = 0; j < 1 + 2 * np && j < 2 * kSmall; ++j) {
@@ -1277,18 +1277,17 @@ __global__ void k_validate_tree(const bvht_node* __restrict__ nodes, const Ctl* 
 
 // Build order triangle array: tris_out[k] = tris_in[index of element k];
 // perm[k] records that index.
-__global__ void k_gather_tris(const float* __restrict__ tin, const float4* __restrict__ ec, uint32_t n,
-                              float* __restrict__ tout, uint32_t* __restrict__ perm, uint32_t* __restrict__ err)
+__global__ void k_gather_tris(const float* __restrict__ tin, const uint32_t* __restrict__ perm, uint32_t n,
+                              float* __restrict__ tout, uint32_t* __restrict__ err)
 {
     uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n)
         return;
-    uint32_t src = __float_as_uint(ec[k].w);
+    uint32_t src = perm[k];
     if (src >= n) {
         atomicOr(err, 16u);
         return;
     }
-    perm[k] = src;
     const float* a = tin + 9 * (size_t)src;
     float* b = tout + 9 * (size_t)k;
 #pragma unroll
@@ -1475,7 +1474,7 @@ __global__ __launch_bounds__(kCtlWG) void k_level_end(BNode* __restrict__ bn, ui
                                                       const uint32_t* __restrict__ child_keys, Ctl* __restrict__ ctl,
                                                       const uint32_t* __restrict__ wgsum, int faithful,
                                                       uint32_t max_leaf, uint32_t hcap, uint32_t rcap,
-                                                      uint32_t* __restrict__ cacc, uint32_t lcap)
+                                                      uint32_t* __restrict__ cacc, uint32_t lcap, uint32_t other)
 {
     __shared__ uint32_t lds[kCtlWG / 64 + 1];
     __shared__ uint32_t base[4];  // splits and large children before this range; level totals
@@ -1553,7 +1552,7 @@ __global__ __launch_bounds__(kCtlWG) void k_level_end(BNode* __restrict__ bn, ui
                         lvl_all[lpos++] = child + side;
                     } else {
                         c.small = rpos;
-                        small_roots[rpos++] = child + side;
+                        small_roots[rpos++] = (child + side) | other;
                     }
                     bn[child + side] = c;
                 }
@@ -1848,29 +1847,36 @@ uint32_t chunk_elems(uint32_t n)
     return c;
 }
 
-void enqueue_level(hipStream_t st, BuildWs& w, int faithful, uint32_t max_leaf, uint32_t chunk)
+// Level `level` of a build: the large nodes' elements are in buffer level % 2
+// and move to the other one.
+void enqueue_level(hipStream_t st, BuildWs& w, uint32_t* perm, uint32_t level, int faithful, uint32_t max_leaf,
+                   uint32_t chunk)
 {
     Ctl* ctl = w.ctl;
     uint32_t* err = &w.ctl->err;
     uint32_t cg = std::min<uint32_t>(kChunkGrid, w.ccap);
+    float4 *ec = w.ec, *elo = w.elo, *oc = w.oc, *olo = w.olo;
+    float2 *ehi = w.ehi, *ohi = w.ohi;
+    if (level & 1u) {
+        std::swap(ec, oc);
+        std::swap(elo, olo);
+        std::swap(ehi, ohi);
+    }
     hipLaunchKernelGGL(k_level_begin, dim3(1 + kInitWGs), dim3(kCtlWG), 0, st, w.bn, w.lvl_all, ctl, w.tasks,
                        w.node_chunk, w.chunks, w.lcap, w.ccap, w.wgsum, chunk, w.bacc, w.child);
-    hipLaunchKernelGGL(k_bins, dim3(cg), dim3(kWG), 0, st, w.ec, w.elo, w.ehi, w.chunks, ctl, w.cacc, w.bacc,
-                       faithful);
+    hipLaunchKernelGGL(k_bins, dim3(cg), dim3(kWG), 0, st, ec, elo, ehi, w.chunks, ctl, w.cacc, w.bacc, faithful);
     hipLaunchKernelGGL(k_decide, dim3(kTaskGrid), dim3(64), 0, st, w.tasks, ctl, w.cacc, w.bacc, w.dec, faithful,
                        max_leaf);
-    hipLaunchKernelGGL(k_part_count, dim3(cg), dim3(kWG), 0, st, w.ec, w.chunks, ctl, w.dec, w.chunk_left);
+    hipLaunchKernelGGL(k_part_count, dim3(cg), dim3(kWG), 0, st, ec, w.chunks, ctl, w.dec, w.chunk_left);
     hipLaunchKernelGGL(k_part_prefix, dim3(kTaskGrid), dim3(64), 0, st, w.node_chunk, ctl, w.chunk_left, w.dec,
                        w.tasks, faithful, max_leaf, w.wgsum);
-    hipLaunchKernelGGL((k_part_scatter<false>), dim3(cg), dim3(kWG), 0, st, w.ec, w.elo, w.ehi, w.chunks, ctl,
-                       w.tasks, w.dec, w.chunk_left, w.kpos, w.sel, w.oc, w.olo, w.ohi, err);
-    hipLaunchKernelGGL((k_part_scatter<true>), dim3(cg), dim3(kWG), 0, st, w.ec, w.elo, w.ehi, w.chunks, ctl,
-                       w.tasks, w.dec, w.chunk_left, w.kpos, w.sel, w.oc, w.olo, w.ohi, err);
-    hipLaunchKernelGGL(k_part_commit, dim3(cg), dim3(kWG), 0, st, w.oc, w.olo, w.ohi, w.chunks, ctl, w.tasks, w.dec,
-                       w.ec, w.elo, w.ehi, w.child);
+    hipLaunchKernelGGL((k_part_scatter<false>), dim3(cg), dim3(kWG), 0, st, ec, elo, ehi, w.chunks, ctl, w.tasks,
+                       w.dec, w.chunk_left, w.kpos, w.sel, oc, olo, ohi, perm, w.child, err);
+    hipLaunchKernelGGL((k_part_scatter<true>), dim3(cg), dim3(kWG), 0, st, ec, elo, ehi, w.chunks, ctl, w.tasks,
+                       w.dec, w.chunk_left, w.kpos, w.sel, oc, olo, ohi, perm, w.child, err);
     hipLaunchKernelGGL(k_level_end, dim3(kLvlWGs), dim3(kCtlWG), 0, st, w.bn, w.lvl_all, w.small_roots,
                        w.level_start, w.tasks, w.dec, w.child, ctl, w.wgsum, faithful, max_leaf, w.hcap, w.rcap,
-                       w.cacc, w.lcap);
+                       w.cacc, w.lcap, level & 1u ? 0u : kOther);
 }
 
 int32_t build_impl(bvht_ctx ctx, float* h_tris, uint32_t n, int faithful, uint32_t max_leaf, bvht_blas* out)
@@ -1891,7 +1897,8 @@ int32_t build_impl(bvht_ctx ctx, float* h_tris, uint32_t n, int faithful, uint32
 
     RC(bvht::host_to_device(ctx, w.tin, h_tris, sizeof(float) * 9 * (size_t)n));
     BVHT_HIP(hipMemsetAsync(b->d_nodes, 0, sizeof(bvht_node) * 2 * (size_t)n, st));
-    hipLaunchKernelGGL(k_init_elems, dim3(nblk(n, 256)), dim3(256), 0, st, w.tin, n, w.ec, w.elo, w.ehi);
+    hipLaunchKernelGGL(k_init_elems, dim3(nblk(n, 256)), dim3(256), 0, st, w.tin, n, w.ec, w.elo, w.ehi,
+                       b->d_perm);
     // root box: update_node_bounds over everything (bvh.rs:537)
     RC(fill(st, w.rootk, kEmptyMin, 3));
     RC(fill(st, w.rootk + 3, kEmptyMax, 3));
@@ -1923,10 +1930,11 @@ int32_t build_impl(bvht_ctx ctx, float* h_tris, uint32_t n, int faithful, uint32
         std::max<uint32_t>(1u, (uint32_t)(1.15 * std::log2(std::max(1.0, (double)n / kSmall))));
     const uint32_t first_levels = forced ? predicted : std::min<uint32_t>(7u, predicted);
     const uint32_t chunk = chunk_elems(n);
+    uint32_t level = 0;
     for (uint32_t batch = 0;; ++batch) {
         uint32_t levels = batch == 0 ? first_levels : std::min<uint32_t>(32u, (forced ? 1u : 2u) << batch);
         for (uint32_t k = 0; k < levels; ++k)
-            enqueue_level(st, w, faithful, max_leaf, chunk);
+            enqueue_level(st, w, b->d_perm, level++, faithful, max_leaf, chunk);
         BVHT_HIP(hipGetLastError());
         BVHT_HIP(hipMemcpyAsync(&h, w.ctl, sizeof h, hipMemcpyDeviceToHost, st));
         BVHT_HIP(hipStreamSynchronize(st));
@@ -1944,9 +1952,9 @@ int32_t build_impl(bvht_ctx ctx, float* h_tris, uint32_t n, int faithful, uint32
     uint32_t R = h.R;
     if (R)
         hipLaunchKernelGGL(k_small_wave, dim3(nblk(R, kSmallWavesPerWG)), dim3(64 * kSmallWavesPerWG), 0, st, w.ec,
-                           w.elo, w.ehi, w.bn, w.small_roots, R, w.snodes, w.pairs, faithful, max_leaf,
+                           w.elo, w.ehi, w.oc, w.olo, w.ohi, b->d_perm, w.bn, w.small_roots, R, w.snodes, w.pairs, faithful, max_leaf,
                            &w.ctl->err);
-    hipLaunchKernelGGL(k_gather_tris, dim3(nblk(n, 256)), dim3(256), 0, st, w.tin, w.ec, n, b->d_tris, b->d_perm,
+    hipLaunchKernelGGL(k_gather_tris, dim3(nblk(n, 256)), dim3(256), 0, st, w.tin, b->d_perm, n, b->d_tris,
                        &w.ctl->err);
     BVHT_HIP(hipGetLastError());
     RC(bvht::mark_for_copy(ctx));

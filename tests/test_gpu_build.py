@@ -289,3 +289,28 @@ def test_refit_across_chunk_boundaries(ctx, orc, tree):
         assert g_used == used
         assert_nodes_equal(got, want, used)
     bvh.close()
+
+
+@pytest.mark.parametrize("mode,max_leaf", [(B.BUILD_REFERENCE, 0), (B.BUILD_SAH, 2), (B.BUILD_SAH, 40)])
+@pytest.mark.parametrize("n", [32, 33, 64, 65, 129, 4097])
+def test_subtrees_end_at_every_level(ctx, orc, n, mode, max_leaf):
+    """Elements change buffers at every level: clusters of 1 to 90 coincident
+    triangles at growing distances end as large leaves, forced median splits
+    and small subtrees after odd and even numbers of levels."""
+    rng = np.random.default_rng(n)
+    sizes = rng.integers(1, 91, n)
+    at = np.cumsum(1.5 ** (np.arange(n) % 40))
+    cluster = np.repeat(np.arange(n), sizes)[:n]
+    mesh = np.tile(unit_triangle(), (n, 1))
+    mesh[:, 0::3] += at[cluster][:, None]
+    mesh[:, 1::3] += (cluster % 7)[:, None]
+    mesh = np.ascontiguousarray(mesh[rng.permutation(n)], np.float32)
+    nodes, used, perm = orc.bvh_build(mesh, mode == B.BUILD_REFERENCE, max_leaf)
+    m = mesh.copy()
+    bvh = B.BvhBuilder(mode, max_leaf, ctx=ctx).build_for(m)
+    g_nodes, g_used, g_tris = bvh.download()
+    assert g_used == used
+    assert_nodes_equal(g_nodes, nodes, used)
+    assert g_tris.tobytes() == perm.tobytes() == m.tobytes()
+    assert mesh[bvh.permutation()].tobytes() == perm.tobytes()
+    bvh.close()
