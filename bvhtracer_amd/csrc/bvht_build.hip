@@ -128,17 +128,28 @@ __device__ __forceinline__ void key_max(uint32_t& k, float f)
         k = max(k, f2key(f));
 }
 
+// The lane exchanges are DPP moves and permlane swaps, not ds_bpermute: 24
+// reductions of 6 steps a chunk in k_part_scatter<true> (1.3M triangles 6,300
+// -> 6,030 us; smaller builds unchanged).
 __device__ __forceinline__ uint32_t wave_min(uint32_t v)
 {
-    for (int o = 32; o > 0; o >>= 1)
-        v = min(v, (uint32_t)__shfl_xor((int)v, o));
-    return v;
+    const uint32_t lane = threadIdx.x & 63u;
+    v = min(v, xor_lane<32>(v, lane));
+    v = min(v, xor_lane<16>(v, lane));
+    v = min(v, xor_lane<8>(v, lane));
+    v = min(v, xor_lane<4>(v, lane));
+    v = min(v, xor_lane<2>(v, lane));
+    return min(v, xor_lane<1>(v, lane));
 }
 __device__ __forceinline__ uint32_t wave_max(uint32_t v)
 {
-    for (int o = 32; o > 0; o >>= 1)
-        v = max(v, (uint32_t)__shfl_xor((int)v, o));
-    return v;
+    const uint32_t lane = threadIdx.x & 63u;
+    v = max(v, xor_lane<32>(v, lane));
+    v = max(v, xor_lane<16>(v, lane));
+    v = max(v, xor_lane<8>(v, lane));
+    v = max(v, xor_lane<4>(v, lane));
+    v = max(v, xor_lane<2>(v, lane));
+    return max(v, xor_lane<1>(v, lane));
 }
 
 // Block-wide reduction of `nv` key values per thread into global atomics:
