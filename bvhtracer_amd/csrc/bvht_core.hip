@@ -1,7 +1,9 @@
 // bvht_core.hip -- context, BLAS storage, refit and the BLAS trace kernels
 // for gfx950 (MI355X).
 //
-// Traversal kernels run one ray per lane (wave64).  Each lane keeps its
+// Traversal kernels run one ray per lane (wave64), but for trees with large
+// leaves (k_trace_group) and small launches over small trees (k_trace_quad),
+// which give a ray 4 to 16 lanes.  In the first form each lane keeps its
 // traversal stack in LDS, laid out slot-major (slot * WG + lane) so the 64
 // lanes of a wave hit 64 distinct banks; entries deeper than the LDS depth
 // spill to a per-ray region of a global buffer.  The visiting order is the
