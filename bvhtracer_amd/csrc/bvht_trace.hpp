@@ -422,11 +422,6 @@ __device__ __forceinline__ uint64_t lanes_of(bool b) { return __builtin_amdgcn_b
 __device__ __forceinline__ bool lane_in(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 __device__ __forceinline__ uint64_t mask_xor1(uint64_t m) { return (m & kEven) << 1 | (m >> 1 & kEven); }
 __device__ __forceinline__ uint64_t mask_xor2(uint64_t m) { return (m & kLow2) << 2 | (m >> 2 & kLow2); }
-// min(a, b) of operands that are never signalling NaNs: no canonicalizes
-__device__ __forceinline__ float min_raw(float a, float b)
-{
-    return __builtin_amdgcn_fmed3f(a, b, __uint_as_float(0xFF800000u));
-}
 
 __device__ __forceinline__ BlasResult traverse_quad(const float4* __restrict__ nodes, const float4* __restrict__ wide,
                                                     const float* __restrict__ tris, const DRay& ray, bool degen,
@@ -459,9 +454,10 @@ __device__ __forceinline__ BlasResult traverse_quad(const float4* __restrict__ n
             // its two bits differ from theirs in the side
             const uint64_t out = lanes_of(((cur >> kPackShift) ^ (pair_bits >> kPackShift)) == 1u);
             uint64_t hit = lanes_of(tmax >= tmin) & lanes_of(tmax > 0.0f) & ~out;
-            // the child's key (meant only where it is hit)
-            float kp = fmaxf(fmaxf(min_raw(nx, dpp_f<kXor1>(nx)), min_raw(ny, dpp_f<kXor1>(ny))),
-                             min_raw(nz, dpp_f<kXor1>(nz)));
+            // the child's key (meant only where it is hit); beside a leaf child
+            // stands a box of NaNs, which fminf passes over
+            float kp = fmaxf(fmaxf(fminf(nx, dpp_f<kXor1>(nx)), fminf(ny, dpp_f<kXor1>(ny))),
+                             fminf(nz, dpp_f<kXor1>(nz)));
             if (degen) {
                 kp = slab_key(make_float4(fminf(lo.x, dpp_f<kXor1>(lo.x)), fminf(lo.y, dpp_f<kXor1>(lo.y)),
                                           fminf(lo.z, dpp_f<kXor1>(lo.z)), 0.0f),

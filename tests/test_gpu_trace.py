@@ -611,3 +611,24 @@ def test_small_launches_over_small_trees(ctx, orc, tree, n):
         bvh.refit(tris)
         orc.bvh_refit(want, used, tris)
     bvh.close()
+
+
+@pytest.mark.parametrize("n", [4096, 9000, 20000])
+def test_quad_ties_without_zero_directions(ctx, orc, n):
+    """Diagonal rays through the corners of a flat grid: up to six triangles
+    at the same t, boxes that tie, leaf children beside interior ones, and no
+    direction component of zero (such a ray in a wave takes the slab tests
+    of the children's boxes).  The first triangle in the binary loop's order
+    is the oracle's, with 1, 8 and 16 rays a wave."""
+    nodes, used, tris = orc.bvh_build(flat_grid(24), False, 2)
+    bvh = upload(ctx, nodes, used, tris)
+    k = np.arange(n)
+    rays = np.zeros(n, B.RAY_DTYPE)
+    rays["d"] = np.stack([1 - 2 * (k & 1), 1 - (k & 2), 1 - (k >> 1 & 2)], 1)
+    corner = np.stack([k // 8 % 25, k // 200 % 25, 0 * k], 1)
+    rays["o"] = corner - rays["d"] * (1 + k % 13)[:, None]
+    rays["tmax"] = np.finfo(np.float32).max
+    ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+    assert_hits_equal(bvh.intersect(rays), ref, f"ties {n}")
+    assert (ref["prim"] != B.MISS).all()
+    bvh.close()
