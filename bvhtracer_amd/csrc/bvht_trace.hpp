@@ -421,6 +421,9 @@ constexpr uint64_t kEven = 0x5555555555555555ull, kLow2 = 0x3333333333333333ull;
 __device__ __forceinline__ uint64_t lanes_of(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 __device__ __forceinline__ bool lane_in(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 __device__ __forceinline__ uint64_t mask_xor1(uint64_t m) { return (m & kEven) << 1 | (m >> 1 & kEven); }
+// Orders a wave's LDS accesses for the compiler where one lane reads what
+// another wrote (LDS serves a wave in order: no instruction).
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
 __device__ __forceinline__ uint64_t mask_xor2(uint64_t m) { return (m & kLow2) << 2 | (m >> 2 & kLow2); }
 
 __device__ __forceinline__ BlasResult traverse_quad(const float4* __restrict__ nodes, const float4* __restrict__ wide,
@@ -492,6 +495,7 @@ __device__ __forceinline__ BlasResult traverse_quad(const float4* __restrict__ n
                 const uint32_t k = __float_as_uint(lane_in((near & leaf) | child) ? neg_inf : key);
                 st[(sp + (lane_in(near & both) ? 1u : 0u)) * 16] = (uint64_t)k << 32 | e;
             }
+            wave_lds_fence();  // the pop's reads come after
             sp += (lane_in(both) ? 1u : 0u) + (lane_in(second) ? 1u : 0u);
             const uint32_t next = lane_in(near) ? ra : rao;
             cur = sp > kQuadSlots - 2 ? kFull : lane_in(pass | pass_o) ? next : kPop;
@@ -535,6 +539,7 @@ __device__ __forceinline__ BlasResult traverse_quad(const float4* __restrict__ n
         }
         if (cur == kDone || cur == kFull)
             break;
+        wave_lds_fence();                 // the next push's writes come after the pop's reads
         __builtin_amdgcn_wave_barrier();  // one loop latch for every lane (see traverse_blas)
     }
     overflow = cur == kFull;
@@ -563,6 +568,7 @@ __device__ __forceinline__ BlasResult trace_quad(const float4* __restrict__ node
                           reinterpret_cast<lds_u64*>(wave) + (lane >> 2), again);
     // (the ballot keeps the binary loop behind the other for the whole wave:
     // both use its LDS)
+    wave_lds_fence();
     if (__builtin_amdgcn_ballot_w64(again) != 0 && again && (lane & 3u) == 0) {
         Stack<kQuadStack, 16> st{wave + (lane >> 2), spill, stride, cap, status};
         uint32_t pairs = 0, tests = 0;
