@@ -38,6 +38,10 @@ int32_t set_error(int32_t code, const char* fmt, ...)
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
     g_error = buf;
+    // a refused hipMalloc is reported here and leaves the device usable: the
+    // launch checks of later calls must not find its error
+    if (code == BVHT_ENOMEM)
+        (void)hipGetLastError();
     return code;
 }
 
@@ -1555,7 +1559,10 @@ void* blas_buffer(bvht_ctx ctx, size_t bytes)
         return p;
     }
     void* p = nullptr;
-    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess)
+        return p;
+    (void)hipGetLastError();  // some callers go on without the buffer
+    return nullptr;
 }
 
 void blas_buffer_release(bvht_ctx ctx, void* p, size_t bytes)

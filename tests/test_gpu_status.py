@@ -173,3 +173,17 @@ def test_camera_schedule_of_another_size_between_graph_replays():
         g.close()
     finally:
         ctx.close()
+
+
+def test_a_refused_allocation_leaves_no_error_behind(ctx):
+    """An allocation that the device cannot give fails by itself: the calls
+    after it, whose launches are checked with hipGetLastError, work."""
+    mesh = scenes.triangle_soup(300, seed=9)
+    for _ in range(2):
+        with pytest.raises(B.BvhtError, match="hipMalloc"):
+            ctx.alloc(1 << 50)
+        bvh = B.BvhBuilder(B.BUILD_SAH, 2, ctx=ctx).build_for(mesh.copy())
+        with pytest.raises(B.BvhtError, match="hipMalloc"):
+            ctx.alloc(1 << 50)
+        bvh.refit()
+        bvh.close()
