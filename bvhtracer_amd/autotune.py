@@ -1,11 +1,17 @@
 """Autotuner for the trace kernels.
 
-Sweeps the trace kernel configurations compiled into libbvht_hip.so
-(workgroup size 64/128/256 lanes x LDS stack depth 8/16/24/32 entries per
-lane; entries beyond the LDS depth spill to HBM) on the caller's own
-workload, and leaves the fastest configuration set on the context.  Results
+Sweeps the library's default and the trace kernel configurations compiled
+into libbvht_hip.so (workgroup size 64/128/256 lanes x LDS stack depth
+8/16/24/32 entries per lane; entries beyond the LDS depth spill to HBM) on the
+caller's own workload, and leaves the fastest set on the context.  Results
 are identical for every configuration (the traversal order is fixed), so the
 tuner only measures time.
+
+A configuration is one of the kernels that give a ray one lane, and while it
+is set every BLAS trace of the context takes that kernel.  The default, (0, 0),
+also has the kernels that give a ray 4 to 16 lanes (trees with large leaves:
+3092 -> 168 us for 409,600 rays; small launches over small trees), so a
+configuration has to beat it by more than TIE to be set.
 """
 import ctypes
 
@@ -13,6 +19,8 @@ from . import _lib as L
 
 WORKGROUPS = (64, 128, 256)
 LDS_DEPTHS = (8, 16, 24, 32)
+DEFAULT = (0, 0)
+TIE = 0.02  # of the default's time: what two timings of one kernel differ by
 
 
 def configurations():
@@ -44,16 +52,19 @@ def time_ms(ctx, run, reps):
 
 
 def tune(ctx, run, reps=3, configs=None, log=None):
-    """Time ``run()`` (which enqueues trace work on ctx's stream) under each
-    configuration; set the fastest on ctx.  Returns (best, {config: ms})."""
+    """Time ``run()`` (which enqueues trace work on ctx's stream) under the
+    default and each configuration, or under ``configs``; set the fastest on
+    ctx.  Returns (best, {config: ms})."""
     table = {}
-    for wg, d in configs or configurations():
+    for wg, d in configs or [DEFAULT] + configurations():
         set_config(ctx, wg, d)
         run()  # warm up this variant
         table[(wg, d)] = time_ms(ctx, run, reps)
         if log:
             log(f"[autotune] wg {wg:3d} lds {d:2d}: {table[(wg, d)]:.4f} ms")
     best = min(table, key=table.get)
+    if DEFAULT in table and table[DEFAULT] <= table[best] * (1.0 + TIE):
+        best = DEFAULT
     set_config(ctx, *best)
     return best, table
 

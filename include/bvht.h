@@ -227,9 +227,12 @@ int32_t bvht_trace_blas_count(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_ra
 
 /* Trace kernel configuration for this context: workgroup size (64, 128 or
  * 256 lanes) and per-lane LDS stack entries (8, 16, 24 or 32; deeper stacks
- * spill to HBM).  wg = 0 restores the default (64 lanes, LDS depth from the
- * tree depth, at most 24).  Results never depend on the configuration; the autotuner
- * (bvhtracer_amd/autotune.py) picks the fastest. */
+ * spill to HBM).  wg = 0 restores the default: 64 lanes, LDS depth from the
+ * tree depth, at most 24, and for BLAS traces of trees with large leaves and
+ * small launches over small trees the kernels that give a ray 4 to 16 lanes,
+ * which a configuration turns off for the context.  Results never depend on
+ * the configuration; the autotuner (bvhtracer_amd/autotune.py) picks the
+ * fastest, the default among them. */
 int32_t bvht_set_trace_config(bvht_ctx ctx, int32_t wg, int32_t lds_depth);
 int32_t bvht_get_trace_config(bvht_ctx ctx, int32_t* wg, int32_t* lds_depth);
 

@@ -632,3 +632,24 @@ def test_quad_ties_without_zero_directions(ctx, orc, n):
     assert_hits_equal(bvh.intersect(rays), ref, f"ties {n}")
     assert (ref["prim"] != B.MISS).all()
     bvh.close()
+
+
+def test_tuning_a_tree_with_large_leaves_keeps_the_default(ctx, orc):
+    """The autotuner's candidates hold the default, whose several lanes a ray
+    are many times faster here than any configuration: tuned or not, the
+    context traces such a tree with them, and the hits are the oracle's."""
+    from bvhtracer_amd import autotune
+
+    nodes, used, tris = orc.bvh_build(scenes.triangle_soup(3000, seed=31), True, 0)
+    bvh = upload(ctx, nodes, used, tris)
+    rays = random_rays(20000, 21)
+    ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+    d_rays, d_hits = ctx.to_device(rays), ctx.alloc(rays.shape[0] * B.HIT_DTYPE.itemsize)
+    try:
+        best, table = autotune.tune(ctx, lambda: bvh.intersect_device(d_rays, rays.shape[0], d_hits), reps=2)
+        assert best == autotune.current(ctx) == autotune.DEFAULT
+        assert set(table) == {autotune.DEFAULT, *autotune.configurations()}
+        assert_hits_equal(bvh.intersect(rays), ref, "tuned")
+    finally:
+        autotune.set_config(ctx, 0, 0)
+    bvh.close()
