@@ -150,16 +150,27 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n)
         p[i] = v;
 }
 
-// parent[] of every used node; interior nodes name their two children.
-__global__ void k_parents(const bvht_node* __restrict__ nodes, uint32_t nodes_used, uint32_t* __restrict__ parent)
+// What an uploaded tree may have and those built here do not: a node with two
+// parents (then it need not be one level below each), child pairs at odd
+// indices.
+constexpr uint32_t kTwoParents = 1u, kOddPairs = 2u;
+
+// parent[] of every used node (BVHT_MISS before); interior nodes name their
+// two children.  Sets kTwoParents and kOddPairs in *flags: here and not in the
+// host's pass over the nodes, where it took as long as the upload (1.3M
+// triangles 6.9 -> 14.2 ms).
+__global__ void k_parents(const bvht_node* __restrict__ nodes, uint32_t nodes_used, uint32_t* __restrict__ parent,
+                          uint32_t* __restrict__ flags)
 {
     uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nodes_used || k == 1)
         return;
     bvht_node nd = nodes[k];
     if (nd.count == 0) {
-        parent[nd.left_first] = k;
-        parent[nd.left_first + 1] = k;
+        const uint32_t a = atomicExch(&parent[nd.left_first], k), b = atomicExch(&parent[nd.left_first + 1], k);
+        const uint32_t f = (a != BVHT_MISS || b != BVHT_MISS ? kTwoParents : 0u) | (nd.left_first & 1u ? kOddPairs : 0u);
+        if (f & ~__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicOr(flags, f);
     }
 }
 
@@ -1379,8 +1390,9 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     bvht_ctx ctx = b->ctx;
     hipStream_t st = ctx->stream;
     uint32_t nb = blocks_for(b->nodes_used, 256);
-    // scratch: [0] depth, then the per-level counts, the count of the nodes
-    // inside chunks, the big-leaf count and the widest leaf
+    // scratch: [0] depth, then (after k_parents' flags in [1]) the per-level
+    // counts, the count of the nodes inside chunks, the big-leaf count and the
+    // widest leaf
     int32_t rc = ensure_scratch(ctx, sizeof(uint32_t) * (2 * (size_t)b->nodes_used + 4));
     if (rc)
         return rc;
@@ -1389,14 +1401,19 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     if (depth == 0) {
         rc = fill_u32(ctx, b->d_parent, BVHT_MISS, b->node_count);
         if (!rc)
-            rc = fill_u32(ctx, d_depth, 0, 1);
+            rc = fill_u32(ctx, d_depth, 0, 2);
         if (rc)
             return rc;
-        hipLaunchKernelGGL(k_parents, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, b->d_parent);
+        hipLaunchKernelGGL(k_parents, dim3(nb), dim3(256), 0, st, b->d_nodes, b->nodes_used, b->d_parent,
+                           d_depth + 1);
         hipLaunchKernelGGL(k_levels, dim3(nb), dim3(256), 0, st, b->nodes_used, b->d_parent, b->d_level, d_depth);
         BVHT_HIP(hipGetLastError());
-        BVHT_HIP(hipMemcpyAsync(&depth, d_depth, 4, hipMemcpyDeviceToHost, st));
+        uint32_t out[2];
+        BVHT_HIP(hipMemcpyAsync(out, d_depth, sizeof out, hipMemcpyDeviceToHost, st));
         BVHT_HIP(hipStreamSynchronize(st));
+        depth = out[0];
+        b->one_parent = !(out[1] & kTwoParents);
+        b->even_pairs = !(out[1] & kOddPairs);
     }
     if (depth == 0 || depth > b->nodes_used)
         return set_error(BVHT_EDEVICE, "BLAS topology: depth %u out of range", depth);
@@ -1523,22 +1540,6 @@ static int32_t validate_nodes(const bvht_node* nodes, uint32_t node_count, uint3
         }
     }
     return BVHT_OK;
-}
-
-// Whether every node has at most one parent, as in every tree this library
-// builds (then a child is exactly one level below its parent).
-static bool one_parent_each(const bvht_node* nodes, uint32_t nodes_used)
-{
-    std::vector<bool> seen(nodes_used, false);
-    for (uint32_t k = 0; k < nodes_used; ++k) {
-        if (k == 1 || nodes[k].count > 0)
-            continue;
-        const uint32_t lf = nodes[k].left_first;
-        if (seen[lf] || seen[lf + 1])
-            return false;
-        seen[lf] = seen[lf + 1] = true;
-    }
-    return true;
 }
 
 constexpr size_t kBlasPoolBytes = size_t(1) << 30;
@@ -2090,9 +2091,6 @@ int32_t bvht_blas_upload(bvht_ctx ctx, const bvht_node* nodes, uint32_t node_cou
     if (rc)
         return rc;
     b->nodes_used = nodes_used;
-    b->one_parent = one_parent_each(nodes, nodes_used);
-    for (uint32_t k = 0; k < nodes_used; ++k)
-        b->even_pairs = b->even_pairs && (k == 1 || nodes[k].count > 0 || (nodes[k].left_first & 1u) == 0);
     rc = host_to_device(ctx, b->d_nodes, nodes, sizeof(bvht_node) * (size_t)node_count);
     if (!rc)
         rc = host_to_device(ctx, b->d_tris, tris, sizeof(float) * 9 * (size_t)n);

@@ -291,6 +291,32 @@ def test_refit_across_chunk_boundaries(ctx, orc, tree):
     bvh.close()
 
 
+@pytest.mark.parametrize("pairs", [(4, 4), (4, 5)])
+def test_uploaded_nodes_with_two_parents(ctx, orc, pairs):
+    """Two branches that name one pair of children, and pairs that overlap by a
+    node (one of them at an odd index): hits and refits are the oracle's."""
+    tris = scenes.triangle_soup(60, seed=3)
+    nodes = np.zeros(8, orc.NODE_DTYPE)
+    for k, (lf, cnt) in {0: (2, 0), 2: (pairs[0], 0), 3: (pairs[1], 0), 4: (0, 20), 5: (20, 20), 6: (40, 20)}.items():
+        nodes["left_first"][k], nodes["count"][k] = lf, cnt
+    used = 6 if pairs[0] == pairs[1] else 7
+    orc.bvh_refit(nodes, used, tris)
+    bvh = upload(ctx, nodes, used, tris)
+    g = np.random.default_rng(5)
+    rays = np.zeros(3000, B.RAY_DTYPE)
+    rays["o"], rays["d"], rays["tmax"] = g.uniform(-6, 6, (3000, 3)), g.standard_normal((3000, 3)), 3e38
+    want = nodes.copy()
+    for frame in (0, 9):
+        moved = scenes.deform_wave(tris, frame, amp=0.5)
+        orc.bvh_refit(want, used, moved)
+        bvh.refit(moved)
+        assert_nodes_equal(bvh.download()[0], want, used)
+        ref = orc.bvh_trace(want, moved, rays.view(orc.RAY_DTYPE), nthreads=8)
+        assert_hits_equal(bvh.intersect(rays), ref, f"pairs {pairs} frame {frame}")
+        assert (ref["prim"] != B.MISS).sum() > 20  # 60 small triangles among 3,000 rays: 57 hits at frame 0
+    bvh.close()
+
+
 @pytest.mark.parametrize("mode,max_leaf", [(B.BUILD_REFERENCE, 0), (B.BUILD_SAH, 2), (B.BUILD_SAH, 40)])
 @pytest.mark.parametrize("n", [32, 33, 64, 65, 129, 4097])
 def test_subtrees_end_at_every_level(ctx, orc, n, mode, max_leaf):
