@@ -71,11 +71,11 @@ __device__ __forceinline__ uint32_t upper_index(const uint32_t* prefix, uint32_t
 // Refit inside the chunks of every BLAS of the batch: entries are (BLAS,
 // chunk) pairs, one workgroup each.
 __global__ __launch_bounds__(kChunkWG) void k_batch_refit_chunks(const BatchBlas* __restrict__ blases,
-                                                                 const uint2* __restrict__ entries)
+                                                                 const uint2* __restrict__ entries, uint32_t stale)
 {
     const uint2 e = entries[blockIdx.x];
     const BatchBlas bb = blases[e.x];
-    refit_chunk(bb.nodes, bb.tris, bb.level, bb.chunks[e.y], bb.chunks[e.y + 1], bb.wide);
+    refit_chunk(bb.nodes, bb.tris, bb.level, bb.chunks[e.y], bb.chunks[e.y + 1], bb.wide, stale);
 }
 
 // The wide records of the BLASes that have them, after their refit: entries
@@ -244,7 +244,6 @@ struct bvht_batch_s {
     uint2* d_refit = nullptr;           // (BLAS, node) of the nodes that cross chunks, grouped by level
     uint2* d_refit_chunks = nullptr;    // (BLAS, chunk) of every chunk
     uint32_t n_refit_chunks = 0;
-    bool any_wide = false;              // some BLAS has wide records
     uint2* d_refit_big = nullptr;       // (BLAS, leaf) of every big leaf
     uint32_t n_refit_big = 0;
     std::vector<uint32_t> refit_off;     // level L occupies [refit_off[L], refit_off[L+1])
@@ -352,7 +351,6 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
         hb[k].level = bl->d_level;
         hb[k].chunks = bl->d_chunks;
         hb[k].wide = bl->d_wide;
-        b->any_wide = b->any_wide || bl->d_wide;
         for (uint32_t c = 0; c < chunk_count(bl->nodes_used); ++c)
             chunks.push_back(make_uint2((uint32_t)k, c));
         max_depth = std::max(max_depth, bl->depth);
@@ -449,8 +447,14 @@ int32_t bvht_batch_refit(bvht_ctx ctx, bvht_batch b)
     if (b->n_refit_big)
         hipLaunchKernelGGL(k_batch_refit_big, dim3(nblk(b->n_refit_big, 4)), dim3(256), 0, ctx->stream, b->d_blases,
                            b->d_refit_big, b->n_refit_big);
+    // the records of all are written if those of one are asked for
+    bool write_wide = false;
+    for (bvht_blas bl : b->blases)
+        write_wide = refit_wide(ctx, bl) || write_wide;
+    for (bvht_blas bl : b->blases)
+        bl->wide_fresh = write_wide;
     hipLaunchKernelGGL(k_batch_refit_chunks, dim3(b->n_refit_chunks), dim3(kChunkWG), 0, ctx->stream, b->d_blases,
-                       b->d_refit_chunks);
+                       b->d_refit_chunks, write_wide ? 0u : 1u);
     // what crosses chunk boundaries: a level of more than kRunWG entries gets a
     // launch of its own; runs of consecutive smaller levels share one
     // single-workgroup launch
@@ -477,7 +481,7 @@ int32_t bvht_batch_refit(bvht_ctx ctx, bvht_batch b)
             flush();
     }
     flush();
-    if (b->any_wide)
+    if (write_wide)
         hipLaunchKernelGGL(k_batch_wide, dim3(b->n_refit_chunks), dim3(kChunkWG), 0, ctx->stream, b->d_blases,
                            b->d_refit_chunks);
     BVHT_HIP(hipGetLastError());

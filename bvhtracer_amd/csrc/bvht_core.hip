@@ -337,9 +337,9 @@ __global__ __launch_bounds__(kChunkWG) void k_refit_chunks(bvht_node* __restrict
                                                            const float* __restrict__ tris,
                                                            const uint32_t* __restrict__ level,
                                                            const uint32_t* __restrict__ chunks,
-                                                           float4* __restrict__ wide)
+                                                           float4* __restrict__ wide, uint32_t stale)
 {
-    refit_chunk(nodes, tris, level, chunks[blockIdx.x], chunks[blockIdx.x + 1], wide);
+    refit_chunk(nodes, tris, level, chunks[blockIdx.x], chunks[blockIdx.x + 1], wide, stale);
 }
 
 // The wide record of every node at even depth, after the node boxes are final.
@@ -1368,17 +1368,30 @@ int32_t device_to_host_beside(bvht_ctx ctx, void* dst, const void* src, size_t b
     return device_to_host_on(ctx, cs, dst, src, bytes);
 }
 
-// Wide records are kept for packed trees of at most kWideTris triangles: every
-// refit writes them again (4 us, for 82k triangles 6), and on larger trees
+// Wide records are kept for packed trees of at most kWideTris triangles:
+// writing them again takes 4 us of a refit (of 9 to 25), and on larger trees
 // launches small enough for traverse_quad are the rarer.
 constexpr uint32_t kWideTris = 1u << 16;
 static size_t wide_bytes(size_t node_count) { return 64 * node_count; }  // the last pair's record ends with them
 
-static void launch_wide(bvht_ctx ctx, bvht_blas b)
+// A refit leaves the records as they are once two refits in a row went by
+// without a launch that asked for them (the models of a TLAS or a batch, which
+// only other kernels trace; with records a refit of 20 to 2,000 triangles took
+// up to 1.6 times what it took before there were any: 720 triangles 9.6 -> 14.9
+// us, without 10.8).  They are then marked as stale on the device, which is
+// what makes a quad launch right whatever the host believes, and the launch
+// that asks next takes a lane a ray until a refit has written them.  They are
+// written by builds and refits only, which a program orders against its traces
+// on every context, never by a trace: another context may be reading them.
+// In a capture they are always written (the graph's later runs ask nobody),
+// and always for a tree that some captured launch reads them of.
+bool refit_wide(bvht_ctx ctx, bvht_blas b)
 {
-    if (b->d_wide)
-        hipLaunchKernelGGL(k_wide, dim3(blocks_for(b->nodes_used, 256)), dim3(256), 0, ctx->stream,
-                           reinterpret_cast<const float4*>(b->d_nodes), b->d_level, b->nodes_used, b->d_wide);
+    if (!b->d_wide)
+        return false;
+    const bool write = ctx->capturing || b->wide_pinned || b->wide_unread++ < 2;
+    b->wide_fresh = write;
+    return write;
 }
 
 // Triangles of a leaf on average (nodes_used counts the dummy: two a leaf).
@@ -1485,8 +1498,10 @@ int32_t launch_refit(bvht_ctx ctx, bvht_blas blas)
     if (blas->n_big_leaves)
         hipLaunchKernelGGL(k_refit_big_leaves, dim3(blocks_for(blas->n_big_leaves, 4)), dim3(256), 0, ctx->stream,
                            blas->d_nodes, blas->d_tris, blas->d_big_leaves, blas->n_big_leaves);
+    const bool write_wide = refit_wide(ctx, blas);
     hipLaunchKernelGGL(k_refit_chunks, dim3(chunk_count(blas->nodes_used)), dim3(kChunkWG), 0, ctx->stream,
-                       blas->d_nodes, blas->d_tris, blas->d_level, blas->d_chunks, blas->d_wide);
+                       blas->d_nodes, blas->d_tris, blas->d_level, blas->d_chunks, blas->d_wide,
+                       write_wide ? 0u : 1u);
     LevelRun run{};
     auto flush = [&]() {
         if (run.levels)
@@ -1510,7 +1525,10 @@ int32_t launch_refit(bvht_ctx ctx, bvht_blas blas)
             flush();
     }
     flush();
-    launch_wide(ctx, blas);
+    if (write_wide)
+        hipLaunchKernelGGL(k_wide, dim3(blocks_for(blas->nodes_used, 256)), dim3(256), 0, ctx->stream,
+                           reinterpret_cast<const float4*>(blas->d_nodes), blas->d_level, blas->nodes_used,
+                           blas->d_wide);
     BVHT_HIP(hipGetLastError());
     return BVHT_OK;
 }
@@ -1663,6 +1681,11 @@ uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n)
     // the tree's bound are the lane-a-ray kernel's)
     if (!blas->d_wide || n > 65536 || ctx->trace_wg > 0 || ctx->tls_on ||
         (ctx->stack_limit && ctx->stack_limit + 1 < blas->depth))
+        return 0;
+    blas->wide_unread = 0;
+    if (ctx->capturing)
+        blas->wide_pinned = true;
+    if (!blas->wide_fresh)
         return 0;
     return n <= 4096 ? 1 : (n <= 16384 ? 8 : 16);
 }

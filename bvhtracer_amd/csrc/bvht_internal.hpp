@@ -1,6 +1,7 @@
 // bvht_internal.hpp -- host-side internals shared by the library's .hip files.
 #pragma once
 
+#include <atomic>
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -120,6 +121,11 @@ struct bvht_blas_s {
     std::vector<uint32_t> level_off;    // level L occupies [level_off[L], level_off[L+1]) of d_level_order
     uint32_t* d_big_leaves = nullptr;   // leaves with more than kBigLeaf triangles (refit a wave each)
     uint32_t n_big_leaves = 0;
+    // Wide records and refits (refit_wide): whether the last refit wrote them,
+    // refits since a launch asked for them, and whether a graph holds one that
+    // does.  Atomic: traces on several contexts set them at once.
+    std::atomic<bool> wide_fresh{true}, wide_pinned{false};
+    std::atomic<uint32_t> wide_unread{0};
     bool one_parent = true;     // no node has two parents (an uploaded tree's may)
     bool even_pairs = true;     // child pairs at even indices (an uploaded tree's may not be)
     uint32_t widest_leaf = 0;   // triangles of the largest leaf (0 if below 64 and leaves are small on average)
@@ -197,6 +203,8 @@ inline uint32_t stack_cap(bvht_ctx ctx, uint32_t need)
 // Rays a wave for a trace of n rays over blas with four lanes a ray, 0 for a
 // lane a ray.
 uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n);
+// Whether the refit of blas enqueued next on ctx is to write its wide records.
+bool refit_wide(bvht_ctx ctx, bvht_blas blas);
 int32_t blas_alloc(bvht_ctx ctx, uint32_t n, uint32_t node_count, bvht_blas* out);
 // Frees the context's BLAS build workspace (bvht_destroy).
 void release_build_ws(bvht_ctx ctx);

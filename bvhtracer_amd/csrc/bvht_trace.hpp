@@ -310,7 +310,8 @@ __device__ __forceinline__ BlasResult traverse_group(const float4* __restrict__ 
 // interior node's its left_first.  A child that is a leaf fills its first
 // slot; the second has ref kNoRef and a box of NaNs, which nothing hits and
 // minima and maxima pass over.  Record 0 belongs to no node (left_first >= 2);
-// its first word is 1 when some node breaks what traverse_quad relies on.
+// its first word is 1 when some node breaks what traverse_quad relies on or the
+// records are older than the boxes (a refit that did not write them).
 constexpr uint32_t kNoRef = 0xFFFFFFFFu;
 constexpr uint32_t kPairRef = 1u << 26;  // side (bit 25) of the record in bits 0..24
 

@@ -81,7 +81,7 @@ __device__ __forceinline__ void refit_big_leaf(bvht_node* __restrict__ nodes, co
     }
 }
 
-// Refit of a chunk of at most kRefitChunk consecutive nodes by one workgroup,
+// Refit of a chunk of consecutive nodes (at most kRefitChunk) by one workgroup,
 // in LDS: every leaf, and every branch whose whole subtree lies in the chunk.
 // Nodes are numbered depth first (a subtree's nodes are consecutive), so a
 // boundary cuts the ancestors of the pair it stands at, and it is put at a
@@ -90,16 +90,22 @@ __device__ __forceinline__ void refit_big_leaf(bvht_node* __restrict__ nodes, co
 // the level passes, where boundaries at every 1,024th node leave 2,004 on 19.
 // Which branches are inside is a property of the tree, kept in bit 31 of
 // `level` (mark_chunk).  Rounds go up the chunk's levels, deepest first, with a
-// barrier between; a branch's children are one level below it.  Bound by
+// barrier between; a branch's children are one level below it.  A tree of at
+// most kRefitChunk nodes is one chunk and has no pass after it (one chunk or
+// chunks of 768: 160 triangles' nodes in 4.4 or 4.2 us, 1,440 in 9.4 or 11.0,
+// 1,960 in 11.4 or 11.3; level passes of all nodes 6.3, 9.7 and 10.7).  Bound by
 // latency and launches up to some 200k triangles (9 us for 81,920, the level
 // passes after it 10; passes of every level took 57), by HBM beyond (16 scenes
 // of 0.9M triangles, 155 MB: 54 us).
-constexpr uint32_t kRefitChunk = 1024;
-constexpr uint32_t kChunkStride = 768, kChunkWindow = kRefitChunk - kChunkStride;
-constexpr uint32_t kChunkWG = 512;
+constexpr uint32_t kRefitChunk = 2048;
+constexpr uint32_t kChunkStride = 768, kChunkWindow = 256;
+constexpr uint32_t kChunkWG = 1024;
 constexpr uint32_t kChunkPer = kRefitChunk / kChunkWG;
 constexpr uint32_t kInChunk = 0x80000000u;
-inline uint32_t chunk_count(uint32_t nodes_used) { return (nodes_used + kChunkStride - 1) / kChunkStride; }
+inline uint32_t chunk_count(uint32_t nodes_used)
+{
+    return nodes_used <= kRefitChunk ? 1u : (nodes_used + kChunkStride - 1) / kChunkStride;
+}
 
 // First node of chunk `chunk`: of the pairs at [768 chunk, + 256) one of the
 // least level (levels without bit 31), the first; by one wave, in every lane.
@@ -183,10 +189,10 @@ __device__ __forceinline__ void mark_chunk(const bvht_node* __restrict__ nodes, 
 
 __device__ __forceinline__ void refit_chunk(bvht_node* __restrict__ nodes, const float* __restrict__ tris,
                                             const uint32_t* __restrict__ level, uint32_t base, uint32_t end,
-                                            float4* __restrict__ wide)
+                                            float4* __restrict__ wide, uint32_t stale)
 {
     if (wide && base == 0 && threadIdx.x == 0)
-        *reinterpret_cast<uint32_t*>(wide) = 0;  // the mark, set again by the records' writing
+        *reinterpret_cast<uint32_t*>(wide) = stale;  // the mark: 1, or 0 if the records are written after this
     __shared__ float box[6][kRefitChunk];
     uint32_t lv[kChunkPer], lf[kChunkPer];
     for (uint32_t j = 0; j < kChunkPer; ++j) {

@@ -5,7 +5,7 @@ import pytest
 
 import bvhtracer_amd as B
 from bvhtracer_amd import autotune, scenes
-from helpers import assert_hits_equal
+from helpers import assert_hits_equal, assert_nodes_equal
 
 pytestmark = pytest.mark.gpu
 
@@ -144,3 +144,47 @@ def test_graph_frame_replays_match_eager(ctx, orc):
     assert_hits_equal(got[sl], oracle_scene_hits(orc, models[0], tlases[0], work[0]["Minv"], rays[sl]),
                       "graph frame vs oracle")
     graph.close()
+
+
+@pytest.mark.parametrize("refits", [1, 2, 3, 5])
+def test_batched_refit_alone_gives_the_oracle_s_nodes_and_hits(ctx, orc, refits):
+    """The batch's refit is the only one: the models' vertices are moved on the
+    device, their nodes then equal the oracle's reverse sweep, and a trace of
+    each model by itself its hits.  Models of one refit chunk and of several,
+    with wide records (packed stacks) and without (leaves of 64 triangles and
+    more), in one batch; after one batched refit, and after so many that the
+    records are no longer written; then once more."""
+    meshes = [scenes.triangle_soup(n, seed=n) for n in (40, 900, 1025, 2500)] + [scenes.triangle_soup(1500, seed=8)]
+    models, tlases, trees = [], [], []
+    for k, mesh in enumerate(meshes):
+        nodes, used, tris = orc.bvh_build(mesh, k == 4, 0 if k == 4 else 1)
+        models.append(B.Bvh.from_arrays(nodes, used, tris, ctx=ctx))
+        tlases.append(B.TlasBuilder(ctx=ctx).build_for([B.SceneObject(0)], [models[-1]]))
+        trees.append([nodes, used, tris])
+    assert trees[4][0]["count"].max() >= 64
+    batch = B.Batch(ctx, tlases)
+    g = np.random.default_rng(refits)
+    rays = np.zeros(2000, B.RAY_DTYPE)
+    rays["o"], rays["d"], rays["tmax"] = g.uniform(-6, 6, (2000, 3)), g.standard_normal((2000, 3)), 3e38
+
+    def check(what):
+        for k, (nodes, used, tris) in enumerate(trees):
+            assert_nodes_equal(models[k].download()[0], nodes, used)
+            ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+            assert_hits_equal(models[k].intersect(rays), ref, f"{what}, model {k}")
+
+    def refit(frame):
+        d_frame = ctx.to_device(np.array([frame], np.uint32))
+        for k, t in enumerate(trees):
+            d_orig = ctx.to_device(t[2])
+            B.deform_wave(ctx, models[k], d_orig, 0.2, 4.0, 0.1, d_frame)
+            ctx.sync()
+            t[2] = models[k].download()[2]
+            orc.bvh_refit(t[0], t[1], t[2])
+        batch.refit()
+
+    for k in range(refits):
+        refit(k + 1)
+    check(f"{refits} batched refits")
+    refit(40)
+    check("and one more")

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import bvhtracer_amd as B
+from bvhtracer_amd import _lib as L
 from bvhtracer_amd import scenes
 from helpers import assert_hits_equal, assert_nodes_equal, comb_tree, oracle_rays_to_product, upload
 
@@ -653,3 +654,112 @@ def test_tuning_a_tree_with_large_leaves_keeps_the_default(ctx, orc):
     finally:
         autotune.set_config(ctx, 0, 0)
     bvh.close()
+
+
+class Moving:
+    """A small tree whose vertices move with every refit, on the device and in
+    the oracle."""
+
+    def __init__(self, ctx, orc, n, max_leaf=2):
+        self.ctx, self.orc = ctx, orc
+        self.nodes, self.used, self.tris = orc.bvh_build(scenes.triangle_soup(n, seed=n), False, max_leaf)
+        self.bvh = upload(ctx, self.nodes, self.used, self.tris)
+        self.rays = random_rays(3000, n)
+        self.step = 0
+        self.aim()
+
+    def aim(self):
+        """Every other ray at a triangle's centroid."""
+        at = self.tris.reshape(-1, 3, 3).mean(1)
+        k = np.arange(0, self.rays.shape[0], 2)
+        self.rays["d"][k] = at[k // 2 % at.shape[0]] - self.rays["o"][k]
+
+    def move(self):
+        self.step += 1
+        self.tris = scenes.deform_wave(self.tris, self.step, amp=0.3)
+        self.orc.bvh_refit(self.nodes, self.used, self.tris)
+        self.aim()
+
+    def hits(self):
+        return self.orc.bvh_trace(self.nodes, self.tris, self.rays.view(self.orc.RAY_DTYPE), nthreads=8)
+
+    def check(self, what, ctx=None):
+        ref = self.hits()
+        d_rays, d_hits = (ctx or self.ctx).to_device(self.rays), (ctx or self.ctx).alloc(24 * self.rays.shape[0])
+        c = ctx or self.ctx
+        L.check(L.lib().bvht_trace_blas(c.handle, self.bvh.handle, d_rays.ptr, self.rays.shape[0], d_hits.ptr, None))
+        assert_hits_equal(d_hits.download(B.HIT_DTYPE, self.rays.shape[0]), ref, what)
+        assert (ref["prim"] != B.MISS).sum() > 300
+
+
+@pytest.mark.parametrize("n", [2, 300, 1023, 1024, 1025, 1400, 5000])
+def test_wide_records_follow_the_refits_that_wrote_them(ctx, orc, n):
+    """Refits stop writing the wide records when two in a row went unread; a
+    trace after any number of refits, and after the ones that write them
+    again, gives the oracle's hits, also on another context.  Trees of one
+    refit chunk (2,048 nodes: 1,024 leaves of one triangle) and of several."""
+    m = Moving(ctx, orc, n, 1)
+    other = B.Context(0)
+    try:
+        for k, refits in enumerate((0, 1, 1, 2, 3, 1, 5, 1, 1)):
+            for _ in range(refits):
+                m.move()
+                m.bvh.refit(m.tris)
+            got = m.bvh.download()[0]
+            assert_nodes_equal(got, m.nodes, m.used)
+            m.check(f"{n}: {refits} refits, step {k}")
+            if k % 2:
+                ctx.sync()
+                m.check(f"{n}: another context, step {k}", other)
+    finally:
+        other.close()
+    m.bvh.close()
+
+
+def test_wide_records_and_captured_launches(ctx, orc):
+    """A captured trace replayed after eager refits, and a captured refit and
+    trace replayed after refits that nobody traced: every replay, and a trace
+    made between capture and first replay, equals the oracle."""
+    m = Moving(ctx, orc, 3000)
+    n = m.rays.shape[0]
+    d_rays, d_hits = ctx.to_device(m.rays), ctx.alloc(24 * n)
+    g = B.Graph.capture(ctx, lambda: m.bvh.intersect_device(d_rays, n, d_hits), keep=(d_rays, d_hits))
+    for k in range(6):
+        m.move()
+        m.bvh.refit(m.tris)
+        d_rays.upload(m.rays)
+        d_hits.upload(np.zeros(n, B.HIT_DTYPE))
+        g.launch()
+        ctx.sync()
+        assert_hits_equal(d_hits.download(B.HIT_DTYPE, n), m.hits(), f"captured trace, refit {k}")
+    g.close()
+    m.bvh.close()
+
+    m = Moving(ctx, orc, 2999)
+    d_rays = ctx.to_device(m.rays)
+    d_tris = ctx.to_device(m.tris)
+    for _ in range(4):
+        m.move()
+        m.bvh.refit(m.tris)
+
+    def enqueue():
+        m.bvh.refit(d_tris)
+        m.bvh.intersect_device(d_rays, n, d_hits)
+
+    g = B.Graph.capture(ctx, enqueue, keep=(d_rays, d_hits, d_tris))
+    m.check("between capture and first replay")
+    for k in range(4):
+        m.move()
+        d_tris.upload(m.tris)
+        d_rays.upload(m.rays)
+        d_hits.upload(np.zeros(n, B.HIT_DTYPE))
+        g.launch()
+        ctx.sync()
+        assert_hits_equal(d_hits.download(B.HIT_DTYPE, n), m.hits(), f"replay {k}")
+        m.check(f"after replay {k}")
+        for _ in range(k):
+            m.move()
+            m.bvh.refit(m.tris)
+        m.check(f"eager refits after replay {k}")
+    g.close()
+    m.bvh.close()
