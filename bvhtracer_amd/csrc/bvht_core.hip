@@ -1637,31 +1637,48 @@ void trace_config(bvht_ctx ctx, uint32_t need, int* wg, int* lds)
 }
 
 // Lanes a ray for a trace of n rays over a tree with large leaves, 0 for the
-// lane-a-ray kernel.  A lane with a leaf of hundreds of triangles holds its
-// wave for all of them, and the longest such wave is the launch.  Measured (us,
-// a lane a ray / 8 lanes / 16 lanes) on the reference builder's trees of soups
-// and icospheres, named with their triangles (mean and largest leaf):
-//   7,500 camera rays: soup 12,583 (52, 707) 1875 / 181 / 92, sphere 12,000
-//     (443, 681) 1453 / 138 / 74, sphere 500 (19, 32) 52 / 13 / 11;
-//   409,600, uneven leaves: soup 12,583 3092 / 243 / 168, 3,000 (24, 191)
-//     1223 / 125 / 109, 800 (12, 65) 271 / 74 / 74, 300 (6.2, 29) 93 / 37 / 50;
-//     1.92M: soup 12,583 2729 / 426 / 486;
-//   409,600, even leaves: sphere 12,000 1920 / 567 / 717, 2,000 (80, 134)
-//     195 / 151 / 216, 1,000 (38, 70) 101 / 109 / 162, 500 47 / 91 / 146.
-// So 16 lanes for launches that leave the chip idle; else a group where the
-// leaves are uneven, 16 lanes while each lane still has two triangles a leaf
-// and the waves have not filled the chip; and 8 for even leaves from a mean of
-// 64, below which a wave's lanes are busy together as they are.
+// lane-a-ray kernel (or quads).  A lane with a leaf of hundreds of triangles
+// holds its wave for all of them, and the longest such wave is the launch.
+// Measured (us, a lane a ray / 8 lanes / 16 lanes; camera rays) on the
+// reference builder's trees, named with their triangles (mean and largest
+// leaf):
+//   uneven leaves, 409,600: soup 12,583 (52, 707) 3092 / 243 / 168, 3,000 (24,
+//     191) 1223 / 125 / 109, 800 (12, 65) 271 / 74 / 74, 300 (6.2, 29) 93 / 37 / 50;
+//     1.05M: 1,000 (12, 81) 1.40 times as fast with 8 lanes, 650 (11, 54) 0.87,
+//     300 (6.5, 28) 0.59; 786,432: all of these faster;
+//   even leaves, 65,536: sphere 180 (6.7, 11) 25 / 20 / 31, 500 (19, 32) - / 27 /
+//     37, 980 (36, 67) 125 / 37 / 51, 3,920 (157, 255) 262 / 66 / 74, and on random
+//     rays 1223 / 117 / 94; 32,768: 980 135 / 24 / 23, 500 19 / 20 / 21;
+//     98,304 and more: below a mean of 64 the gain turns into a loss (1.05M: 980
+//     212 / 430); 2,000 (80, 136) 262,144 198 / 164, 786,432 1.04 times as fast, 1.05M
+//     455 / 619; 1.05M: 5,780 (222, 387) 0.80 times, 8,000 (320, 530) 1.04, 11,520
+//     (480, 710) 1.41, 2.1M 0.84, 0.89 and 1.06;
+//   one leaf for all rays: 6 triangles, 16,384 3.9 / 3.3 / 3.4, 65,536 4.3 / 4.2 / 6.5;
+//     64, 98,304 20.4 / 13.3, 196,608 0.99 times, 262,144 27.7 / 31.0.
+// So 16 lanes while all their waves are resident at once (32,768 rays), beyond
+// that where lanes find enough triangles in a leaf; 8 for the rest; and a lane
+// a ray where its waves keep their lanes busy by themselves: even and small
+// leaves, one leaf, and from 786,432 rays on all but the largest leaves.
+// (Random rays would gain there, 2,000 (80, 136) at 1.05M 1726 / 737, but a
+// launch does not tell which it has, and the camera's would lose.)
 static int leaf_group(bvht_blas b, uint32_t n)
 {
     const uint32_t mean = mean_leaf(b);
     if (mean < kGroupLeaf)
         return 0;
+    const bool uneven = b->widest_leaf >= 4 * mean;
+    if (!uneven && mean < 64) {
+        if (n > (mean < 8 ? 16384u : 65536u))
+            return 0;
+        return n <= 32768 ? 16 : 8;
+    }
     if (n <= 65536)
         return 16;
-    if (b->widest_leaf >= 4 * mean)
-        return mean >= 24 && n <= (1u << 20) ? 16 : 8;
-    return mean >= 64 ? 8 : 0;
+    if (b->nodes_used <= 2 && n > (1u << 17))
+        return 0;
+    if (n > 3u << 18 && mean < (uneven ? 12u : 400u))
+        return 0;
+    return uneven && mean >= 24 && n <= (1u << 20) ? 16 : 8;
 }
 
 // Four lanes a ray where the launch is as long as its longest rays: a quad's

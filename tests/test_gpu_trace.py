@@ -763,3 +763,21 @@ def test_wide_records_and_captured_launches(ctx, orc):
         m.check(f"eager refits after replay {k}")
     g.close()
     m.bvh.close()
+
+
+@pytest.mark.parametrize("mesh,n", [("sphere980", 32768), ("sphere980", 32769), ("sphere980", 65537), ("leaf7", 16384), ("leaf7", 16385),
+                                    ("leaf8", 65536), ("leaf70", 131072), ("leaf70", 131073), ("soup300", 786432),
+                                    ("soup300", 786433), ("soup1100", 786433), ("sphere2000", 786433)])
+def test_lanes_a_ray_change_with_leaves_and_rays(ctx, orc, mesh, n):
+    """Both sides of every line between 16 lanes a ray, 8 and one (even and
+    uneven leaves, one leaf for all rays, counts of 16,384 to
+    786,433 rays): the oracle's hits."""
+    kind, tri = mesh.rstrip("0123456789"), int(mesh.lstrip("abcdefghijklmnopqrstuvwxyz"))
+    tris = scenes.icosphere(round((tri / 20) ** 0.5), radius=4.0) if kind == "sphere" else scenes.triangle_soup(tri, seed=2)
+    nodes, used, tris = (*leaf_tree(tris), tris) if kind == "leaf" else orc.bvh_build(tris, True, 0)
+    bvh = upload(ctx, nodes, used, tris)
+    rays = random_rays(n, 78)
+    ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+    assert_hits_equal(bvh.intersect(rays), ref, f"{mesh} {n}")
+    assert (ref["prim"] != B.MISS).sum() > 5
+    bvh.close()
