@@ -1691,12 +1691,17 @@ static int leaf_group(bvht_blas b, uint32_t n)
 //   65,536         135 / 107 / 105 / 110    58 / 155 / 57 / 46
 //   160,000        158 / 167 / 114 / 117    58 / 323 / 78 / 64
 // and the same order on random rays (64 rays 88 / 51 and 36 / 22, 65,536 298 /
-// 204 and 81 / 61, 200,000 278 / 304 and 90 / 103 with 1 and 16).
+// 204 and 81 / 61, 200,000 278 / 304 and 90 / 103 with 1 and 16).  Over a few
+// dozen triangles a lane's walk is short and the waves come first: sphere of 80,
+// 4,096 camera rays 17.0 / 19.6 / 15.6 / 15.3, 65,536 16.6 / - / 26.6 / 19.4; of 20,
+// 32,768 12.2 / - / 13.4 / 11.6; soup of 4 no gain at any count; of 180, 65,536
+// 20.2 / - / 24.5 / 19.9.
 uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n)
 {
     // (the autotuner's configurations, the wave order and a stack limit below
     // the tree's bound are the lane-a-ray kernel's)
-    if (!blas->d_wide || n > 65536 || ctx->trace_wg > 0 || ctx->tls_on ||
+    const bool few = blas->n_tris < 96;
+    if (!blas->d_wide || blas->n_tris < 8 || n > (few ? 32768u : 65536u) || ctx->trace_wg > 0 || ctx->tls_on ||
         (ctx->stack_limit && ctx->stack_limit + 1 < blas->depth))
         return 0;
     blas->wide_unread = 0;
@@ -1704,7 +1709,7 @@ uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n)
         blas->wide_pinned = true;
     if (!blas->wide_fresh)
         return 0;
-    return n <= 4096 ? 1 : (n <= 16384 ? 8 : 16);
+    return n <= (few ? 2048u : 4096u) ? 1 : (!few && n <= 16384 ? 8 : 16);
 }
 
 int32_t launch_trace_blas(bvht_ctx ctx, bvht_blas blas, const bvht_ray* d_rays, uint32_t n,

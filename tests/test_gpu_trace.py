@@ -781,3 +781,18 @@ def test_lanes_a_ray_change_with_leaves_and_rays(ctx, orc, mesh, n):
     assert_hits_equal(bvh.intersect(rays), ref, f"{mesh} {n}")
     assert (ref["prim"] != B.MISS).sum() > 5
     bvh.close()
+
+
+@pytest.mark.parametrize("tri,n", [(7, 900), (8, 2048), (8, 2049), (95, 2049), (95, 32768), (95, 32769), (96, 4097),
+                                   (96, 65536), (96, 65537)])
+def test_few_triangles_and_few_rays(ctx, orc, tri, n):
+    """Both sides of the lines between four lanes a ray and one, and between 1,
+    8 and 16 rays a wave, over trees of a few dozen triangles."""
+    nodes, used, tris = orc.bvh_build(scenes.triangle_soup(tri, seed=6), False, 1)
+    bvh = upload(ctx, nodes, used, tris)
+    rays = random_rays(n, 61)
+    rays["d"] = tris.reshape(-1, 3, 3).mean(1)[np.arange(n) % tri] + f32(0.3) * rays["d"] - rays["o"]
+    ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+    assert_hits_equal(bvh.intersect(rays), ref, f"{tri} triangles, {n} rays")
+    assert (ref["prim"] != B.MISS).sum() > n // 20
+    bvh.close()
