@@ -150,11 +150,12 @@ __global__ void k_batch_bounds(const BatchScene* __restrict__ scenes, const uint
     object_bounds(sc.objects, sc.blases, sc.bounds, sc.rows_w, k - obj_prefix[s]);
 }
 
+template <bool WAVE>
 __global__ __launch_bounds__(kRebuildWG) void k_batch_rebuild(const BatchScene* __restrict__ scenes)
 {
     BatchScene sc = scenes[blockIdx.x];
     extern __shared__ float rebuild_lds[];
-    tlas_rebuild_block(sc.bounds, sc.n_obj, sc.nodes_w, sc.list, sc.meta, rebuild_lds);
+    tlas_rebuild_block<WAVE>(sc.bounds, sc.n_obj, sc.nodes_w, sc.list, sc.meta, rebuild_lds);
 }
 
 template <int WG, int LDS_DEPTH, int RPI>
@@ -248,7 +249,7 @@ struct bvht_batch_s {
     uint32_t n_refit_big = 0;
     std::vector<uint32_t> refit_off;     // level L occupies [refit_off[L], refit_off[L+1])
     uint32_t* d_obj_prefix = nullptr;
-    uint32_t total_nodes = 0, total_objs = 0;
+    uint32_t total_nodes = 0, total_objs = 0, max_objs = 0;
     size_t rebuild_lds = 0;  // dynamic LDS of k_batch_rebuild: the largest scene's list
     uint32_t cap = 0;  // traversal stack bound: max over scenes of (objects - 1) + (BLAS depth - 1)
     // trace tables (bvht_batch_set_rays)
@@ -332,6 +333,7 @@ int32_t bvht_batch_create(bvht_ctx ctx, const bvht_tlas* scenes, uint32_t n_scen
         d.list = t->d_list;
         d.meta = t->d_meta;
         d.n_obj = t->n;
+        b->max_objs = std::max(b->max_objs, t->n);
         b->rebuild_lds = std::max(b->rebuild_lds, rebuild_lds_bytes(t->n));
         d.pad = 0;
         obj_prefix[s + 1] = obj_prefix[s] + t->n;
@@ -500,8 +502,8 @@ int32_t bvht_batch_rebuild(bvht_ctx ctx, bvht_batch b)
     }
     hipLaunchKernelGGL(k_batch_bounds, dim3(nblk(b->total_objs, 64)), dim3(64), 0, ctx->stream, b->d_scenes,
                        b->d_obj_prefix, (uint32_t)b->scenes.size());
-    hipLaunchKernelGGL(k_batch_rebuild, dim3((uint32_t)b->scenes.size()), dim3(kRebuildWG), b->rebuild_lds,
-                       ctx->stream, b->d_scenes);
+    hipLaunchKernelGGL(b->max_objs <= 64 ? k_batch_rebuild<true> : k_batch_rebuild<false>,
+                       dim3((uint32_t)b->scenes.size()), dim3(kRebuildWG), b->rebuild_lds, ctx->stream, b->d_scenes);
     BVHT_HIP(hipGetLastError());
     return BVHT_OK;
 }

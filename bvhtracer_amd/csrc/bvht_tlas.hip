@@ -33,11 +33,12 @@ __global__ void k_object_bounds(const bvht_instance* __restrict__ objs, uint32_t
         object_bounds(objs, blases, bounds, rows, i);
 }
 
+template <bool WAVE>
 __global__ __launch_bounds__(kRebuildWG) void k_tlas_rebuild(const float* __restrict__ bounds, uint32_t n,
                                                              bvht_tnode* nodes, int32_t* list, uint32_t* meta)
 {
     extern __shared__ float rebuild_lds[];
-    tlas_rebuild_block(bounds, n, nodes, list, meta, rebuild_lds);
+    tlas_rebuild_block<WAVE>(bounds, n, nodes, list, meta, rebuild_lds);
 }
 
 template <int WG, int LDS_DEPTH, bool STATS, bool PACKED>
@@ -180,8 +181,8 @@ int32_t refresh(bvht_tlas t)
 
 int32_t rebuild(bvht_tlas t, bool read_depth)
 {
-    hipLaunchKernelGGL(k_tlas_rebuild, dim3(1), dim3(kRebuildWG), rebuild_lds_bytes(t->n), t->ctx->stream,
-                       t->d_bounds, t->n, t->d_nodes, t->d_list, t->d_meta);
+    hipLaunchKernelGGL(t->n <= 64 ? k_tlas_rebuild<true> : k_tlas_rebuild<false>, dim3(1), dim3(kRebuildWG),
+                       rebuild_lds_bytes(t->n), t->ctx->stream, t->d_bounds, t->n, t->d_nodes, t->d_list, t->d_meta);
     BVHT_HIP(hipGetLastError());
     if (read_depth) {
         uint32_t meta[3];

@@ -188,3 +188,24 @@ def test_batched_refit_alone_gives_the_oracle_s_nodes_and_hits(ctx, orc, refits)
     check(f"{refits} batched refits")
     refit(40)
     check("and one more")
+
+
+@pytest.mark.parametrize("counts", [(1, 2, 64), (64, 65, 300), (3, 2049)])
+def test_batched_rebuild_of_few_and_many_objects(ctx, orc, counts):
+    """Scenes of one wave's objects, of LDS lists and of global lists in one
+    batched rebuild: every TLAS equals the oracle's."""
+    nodes, used, tris = orc.bvh_build(scenes.icosphere(3, radius=2.0), False, 2)
+    model = B.Bvh.from_arrays(nodes, used, tris, ctx=ctx)
+    tlases, wants = [], []
+    for n in counts:
+        M, Minv = scenes.random_affines(n, n, trans_range=40.0)
+        objs = [B.SceneObject(0, M[k], Minv[k]) for k in range(n)]
+        tlases.append(B.TlasBuilder(ctx=ctx).build_for(objs, [model]))
+        bounds = np.stack([np.concatenate(orc.instance_bounds(o.m, nodes[0]["bmin"], nodes[0]["bmax"])) for o in objs])
+        wants.append(orc.tlas_build(bounds))
+    batch = B.Batch(ctx, tlases)
+    batch.rebuild()
+    ctx.sync()
+    for n, t, (want, want_used) in zip(counts, tlases, wants):
+        got, got_used = t.download()
+        assert got_used == want_used and got.tobytes() == want.tobytes(), n
