@@ -417,3 +417,31 @@ def test_gradient_descent_lowers_the_loss(ctx, scene):
         mesh.update(normals=True)
     assert losses[-1] < losses[0] * 2.0 / 3.0, losses
     mesh.close()
+
+
+@pytest.mark.parametrize("freq,counts", [(2, (1, 2049, 32768, 32769)), (16, (1, 4096, 4097, 16385, 65536, 65537)),
+                                         (57, (65536, 65537)), (58, (65536, 262144, 262145, 262144, 500001, 262145))])
+def test_small_forwards_bitwise_equal_the_oracle(ctx, orc, freq, counts):
+    """Forwards that take four lanes a ray (up to 65,536 rays over up to 65,536
+    faces; 80, 5,120, 64,980 and 67,280 here) and those too small for a wave
+    order (up to 262,144 rays), on both sides of each line and in turn on one
+    mesh: hits and image are the oracle's bit for bit, also after the vertices
+    moved."""
+    w = scenes.diff_workload(freq, width=W, n_cameras=2)
+    mesh, _ = make_mesh(ctx, w["V"], w["F"])
+    rays = gpu_rays(ctx, w["cameras"], W).download(B.RAY_DTYPE, 2 * W * W)
+    rays = rays[np.random.default_rng(freq).permutation(rays.shape[0])]
+    d_rays = ctx.to_device(rays)
+    for step, V in enumerate((w["V"], scenes.radial_perturb(w["V"], 0.03, seed=4))):
+        if step:
+            mesh.set_vertices(V, normals=True)
+        vid, nodes, _, tris = vid_of(mesh)
+        _, N = mesh.download()
+        ref_h, ref_img = orc.diff_forward(nodes, tris, vid, N, w["Minv"], w["light"], rays.view(orc.RAY_DTYPE), 8)
+        assert (ref_h["prim"] != B.MISS).sum() > rays.shape[0] // 4
+        for n in counts:
+            d_hits, d_img = ctx.alloc(24 * n), ctx.alloc(8 * n)
+            B.trace_forward(mesh, w["Minv"], w["light"], d_rays, n, d_hits, d_img)
+            assert_hits_equal(d_hits.download(B.HIT_DTYPE, n), ref_h[:n], f"{freq}, {n} rays, step {step}")
+            assert d_img.download(np.float32, 2 * n).tobytes() == ref_img[:n].tobytes()
+    mesh.close()

@@ -386,3 +386,25 @@ def test_tlas_wave_schedule_keeps_hits(orc):
         assert d_hits.download(B.HIT_DTYPE, n).tobytes() == want.tobytes()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n", [2, 64, 65, 70, 300, 2048, 2049])
+@pytest.mark.parametrize("near", [0, 1])
+def test_rebuild_without_a_finite_candidate_is_refused(ctx, orc, n, near):
+    """Objects so far apart that every area overflows (all of them, or all but
+    a near pair, which is merged first): an error from each of the three merge
+    loops, and the next TLAS is as it should be."""
+    nodes, used, tris = orc.bvh_build(scenes.icosphere(2, radius=1.0), False, 2)
+    model = B.Bvh.from_arrays(nodes, used, tris, ctx=ctx)
+    at = np.outer(np.arange(n + near), np.full(3, 1e30)).astype(np.float32)
+    if near:
+        at[1] = (3.0, 0.0, 0.0)
+    M, Minv = translated(at)
+    objs = [B.SceneObject(0, M[k], Minv[k]) for k in range(n + near)]
+    with pytest.raises(B.BvhtError, match="no finite merge candidate"):
+        B.TlasBuilder(ctx=ctx).build_for(objs, [model])
+    M, Minv = scenes.random_affines(n, 5, trans_range=30.0)
+    objs = [B.SceneObject(0, M[k], Minv[k]) for k in range(n)]
+    want, want_used = oracle_tlas(orc, [(nodes, tris)], objs)
+    got, got_used = B.TlasBuilder(ctx=ctx).build_for(objs, [model]).download()
+    assert got_used == want_used and got.tobytes() == want.tobytes()

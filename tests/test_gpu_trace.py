@@ -796,3 +796,78 @@ def test_few_triangles_and_few_rays(ctx, orc, tri, n):
     assert_hits_equal(bvh.intersect(rays), ref, f"{tri} triangles, {n} rays")
     assert (ref["prim"] != B.MISS).sum() > n // 20
     bvh.close()
+
+
+@pytest.fixture
+def lane_a_ray(ctx):
+    """A trace configuration is set: every BLAS trace gives a ray one lane."""
+    from bvhtracer_amd import autotune
+
+    autotune.set_config(ctx, 64, 8)
+    yield
+    autotune.set_config(ctx, 0, 0)
+
+
+@pytest.mark.parametrize("left_count", [63, 64, 65])
+def test_stack_entry_packing_boundary_with_a_lane_a_ray(ctx, orc, lane_a_ray, left_count):
+    """The same trees in the kernel that packs a leaf into its stack entry (by
+    default their large leaves take a group of lanes a ray)."""
+    test_stack_entry_packing_boundary(ctx, orc, left_count)
+
+
+def test_deep_tree_uses_spill_with_a_lane_a_ray(ctx, orc, lane_a_ray):
+    """142 entries beyond the LDS stack (by default quads hand such rays on)."""
+    test_deep_tree_uses_spill(ctx, orc)
+
+
+def comb_of_large_leaves(levels, per):
+    """comb_tree with `per` triangles a leaf, one behind the other."""
+    nodes, used, tris = comb_tree(levels)
+    many = np.repeat(tris, per, axis=0)
+    many[:, 0::3] += (np.arange(levels * per) % per)[:, None].astype(f32) / f32(2 * per)
+    leaf = nodes["count"] > 0
+    nodes["left_first"][leaf] *= per
+    nodes["count"][leaf] *= per
+    return nodes, used, many
+
+
+@pytest.mark.parametrize("n", [3000, 40000])
+def test_large_leaves_in_a_deep_tree_spill(ctx, orc, n):
+    """A comb of 120 levels with 9 triangles a leaf: groups of 16 lanes (3,000
+    rays) and of 8 (40,000) push 118 entries, 54 beyond their LDS stack."""
+    nodes, used, tris = comb_of_large_leaves(120, 9)
+    orc.bvh_refit(nodes, used, tris)
+    assert orc.bvh_depth(nodes) == 120
+    bvh = upload(ctx, nodes, used, tris)
+    k = np.arange(n)
+    rays = np.zeros(n, B.RAY_DTYPE)
+    rays["o"] = np.stack([np.full(n, -5.0), (k % 64) / 64.0 - 0.5, (k // 64 % 64) / 64.0 - 0.5], 1)
+    rays["d"] = np.stack([np.ones(n), np.full(n, 1e-3), np.full(n, -1e-3)], 1)
+    rays["o"][2::3] += f32([130.0, 0.0, 0.0])  # from the other end
+    rays["d"][2::3, 0] = -1.0
+    rays["tmax"] = np.where(k % 2 == 0, np.finfo(np.float32).max, f32(4.0))
+    ref = orc.bvh_trace(nodes, tris, rays.view(orc.RAY_DTYPE), nthreads=8)
+    assert_hits_equal(bvh.intersect(rays), ref, f"deep large leaves {n}")
+    assert n // 3 < (ref["prim"] != B.MISS).sum() < n
+    bvh.close()
+
+
+@pytest.mark.parametrize("tree", ["quads", "lanes16", "lanes8"])
+@pytest.mark.parametrize("count", [0, 1, 4095, 4999, 5000, 70000])
+def test_ray_count_on_the_device(ctx, orc, tree, count):
+    """bvht_trace_blas_count where several lanes take a ray: the first *d_count
+    rays (at most max_n) are traced, the other hits are left alone."""
+    max_n = 40000 if tree == "lanes8" else 5000
+    nodes, used, tris = orc.bvh_build(scenes.icosphere(7, radius=4.0), tree != "quads", 0 if tree != "quads" else 2)
+    bvh = upload(ctx, nodes, used, tris)
+    rays = random_rays(max_n, 12)
+    d_rays, d_hits = ctx.to_device(rays), ctx.alloc(24 * max_n)
+    d_hits.upload(np.full(24 * max_n, 0xA5, np.uint8))
+    d_count = ctx.to_device(np.array([count], np.uint32))
+    L.check(L.lib().bvht_trace_blas_count(ctx.handle, bvh.handle, d_rays.ptr, d_count.ptr, max_n, d_hits.ptr, None))
+    got = d_hits.download(B.HIT_DTYPE, max_n)
+    done = min(count, max_n)
+    ref = orc.bvh_trace(nodes, tris, rays[:done].view(orc.RAY_DTYPE), nthreads=8)
+    assert_hits_equal(got[:done], ref, f"{tree}, {count} of {max_n}")
+    assert (got[done:].view(np.uint8) == 0xA5).all()
+    bvh.close()
