@@ -1412,6 +1412,9 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
     uint32_t* d_depth = static_cast<uint32_t*>(ctx->scratch);
     uint32_t depth = known_depth;
     if (depth == 0) {
+        b->d_parent = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)b->node_count));
+        if (!b->d_parent)
+            return set_error(BVHT_ENOMEM, "device allocation for a BLAS of %u triangles failed", b->n_tris);
         rc = fill_u32(ctx, b->d_parent, BVHT_MISS, b->node_count);
         if (!rc)
             rc = fill_u32(ctx, d_depth, 0, 2);
@@ -1606,11 +1609,10 @@ int32_t blas_alloc(bvht_ctx ctx, uint32_t n, uint32_t node_count, bvht_blas* out
     b->node_count = node_count;
     b->d_nodes = static_cast<bvht_node*>(blas_buffer(ctx, sizeof(bvht_node) * (size_t)node_count));
     b->d_tris = static_cast<float*>(blas_buffer(ctx, sizeof(float) * 9 * (size_t)n));
-    b->d_parent = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)node_count));
     b->d_level = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)node_count));
     b->d_level_order = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (size_t)node_count));
     b->d_chunks = static_cast<uint32_t*>(blas_buffer(ctx, sizeof(uint32_t) * (chunk_count(node_count) + 1)));
-    bool ok = b->d_nodes && b->d_tris && b->d_parent && b->d_level && b->d_level_order && b->d_chunks;
+    bool ok = b->d_nodes && b->d_tris && b->d_level && b->d_level_order && b->d_chunks;
     if (!ok) {
         bvht_blas_destroy(b);
         return set_error(BVHT_ENOMEM, "device allocation for a BLAS of %u triangles failed", n);
