@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kWG) void k_range_box(const float4* __restrict__ el
 
 // Centroid range of elements [0, n) into keys[6] = {min xyz, max xyz}: the
 // root's (find_best_split_plane, bvh.rs:338-344).  The children's come out of
-// part_commit_chunk, which reads every element of a split node anyway.
+// part_scatter_chunk, which moves every element of a split node anyway.
 __global__ __launch_bounds__(kWG) void k_centroid_root(const float4* __restrict__ ec, uint32_t n,
                                                        uint32_t* __restrict__ keys)
 {
