@@ -94,9 +94,9 @@ __device__ __forceinline__ void refit_big_leaf(bvht_node* __restrict__ nodes, co
 // most kRefitChunk nodes is one chunk and has no pass after it (one chunk or
 // chunks of 768: 160 triangles' nodes in 4.4 or 4.2 us, 1,440 in 9.4 or 11.0,
 // 1,960 in 11.4 or 11.3; level passes of all nodes 6.3, 9.7 and 10.7).  Bound by
-// latency and launches up to some 200k triangles (9 us for 81,920, the level
-// passes after it 10; passes of every level took 57), by HBM beyond (16 scenes
-// of 0.9M triangles, 155 MB: 54 us).
+// latency and launches up to some 200k triangles (8.9 us for 81,920, the level
+// passes after it 10.3), by HBM beyond (16 scenes of 0.9M triangles, 155 MB: 62
+// us; 54 where no chunk has more than 1,024 nodes, with 512 threads).
 constexpr uint32_t kRefitChunk = 2048;
 constexpr uint32_t kChunkStride = 768, kChunkWindow = 256;
 constexpr uint32_t kChunkWG = 1024;

@@ -255,8 +255,9 @@ int32_t bvht_set_stack_limit(bvht_ctx ctx, uint32_t max_entries);
  * default; the _count variants and traces that collect statistics are never
  * reordered.  While it is on, BLAS traces give a ray one lane, also over trees
  * with large leaves, where the default's several lanes are many times faster:
- * turn it on for scenes, or for the traces that gain.  A call that would have to grow the order buffers while a graph
- * captured on the context lives is refused (BVHT_EINVAL). */
+ * turn it on for scenes, or for the traces that gain.  A call that would have
+ * to grow the order buffers while a graph captured on the context lives is
+ * refused (BVHT_EINVAL). */
 int32_t bvht_set_wave_schedule(bvht_ctx ctx, int32_t enable);
 
 /* ---- frame loop ------------------------------------------------------- */
