@@ -1648,7 +1648,7 @@ void trace_config(bvht_ctx ctx, uint32_t need, int* wg, int* lds)
 //     191) 1223 / 125 / 109, 800 (12, 65) 271 / 74 / 74, 300 (6.2, 29) 93 / 37 / 50;
 //     1.05M: 1,000 (12, 81) 1.40 times as fast with 8 lanes, 650 (11, 54) 0.87,
 //     300 (6.5, 28) 0.59; 786,432: all of these faster;
-//   even leaves, 65,536: sphere 180 (6.7, 11) 25 / 20 / 31, 500 (19, 32) - / 27 /
+//   even leaves, 65,536: sphere 180 (6.7, 11) 25 / 20 / 31 (quads 12), 500 (19, 32) - / 27 /
 //     37, 980 (36, 67) 125 / 37 / 51, 3,920 (157, 255) 262 / 66 / 74, and on random
 //     rays 1223 / 117 / 94; 32,768: 980 135 / 24 / 23, 500 19 / 20 / 21;
 //     98,304 and more: below a mean of 64 the gain turns into a loss (1.05M: 980
@@ -1707,10 +1707,10 @@ uint32_t quad_rays(bvht_ctx ctx, bvht_blas blas, uint32_t n)
         (ctx->stack_limit && ctx->stack_limit + 1 < blas->depth))
         return 0;
     blas->wide_unread = 0;
-    if (ctx->capturing)
-        blas->wide_pinned = true;
     if (!blas->wide_fresh)
         return 0;
+    if (ctx->capturing)
+        blas->wide_pinned = true;
     return n <= (few ? 2048u : 4096u) ? 1 : (!few && n <= 16384 ? 8 : 16);
 }
 
