@@ -323,13 +323,19 @@ __global__ __launch_bounds__(256) void k_chunk_starts(const uint32_t* __restrict
         chunks[c] = at;
 }
 
-__global__ __launch_bounds__(kChunkWG) void k_mark_chunks(const bvht_node* __restrict__ nodes,
-                                                          const uint32_t* __restrict__ chunks,
+// (A tree of one chunk has its two starts written here: a launch fewer.)
+__global__ __launch_bounds__(kChunkWG) void k_mark_chunks(const bvht_node* __restrict__ nodes, uint32_t nodes_used,
+                                                          uint32_t* __restrict__ chunks,
                                                           uint32_t* __restrict__ level, float4* __restrict__ wide)
 {
     if (wide && blockIdx.x == 0 && threadIdx.x == 0)
         *reinterpret_cast<uint32_t*>(wide) = 0;  // the records' mark
-    mark_chunk(nodes, chunks[blockIdx.x], chunks[blockIdx.x + 1], level);
+    const bool one = gridDim.x == 1;
+    if (one && threadIdx.x == 0) {
+        chunks[0] = 0;
+        chunks[1] = nodes_used;
+    }
+    mark_chunk(nodes, one ? 0 : chunks[blockIdx.x], one ? nodes_used : chunks[blockIdx.x + 1], level);
 }
 
 // Bvh::refit inside the chunks (see refit_chunk); the level passes follow.
@@ -1443,11 +1449,12 @@ int32_t compute_blas_topology(bvht_blas b, const bvht_node*, uint32_t known_dept
         b->d_wide = static_cast<float4*>(blas_buffer(ctx, wide_bytes(b->node_count)));  // (none: no quads)
     // (a tree with shared nodes keeps to the level passes)
     const uint32_t n_chunks = chunk_count(b->nodes_used);
-    hipLaunchKernelGGL(k_chunk_starts, dim3(blocks_for(n_chunks + 1, 4)), dim3(256), 0, st, b->d_level, b->nodes_used,
-                       n_chunks, b->d_chunks);
+    if (n_chunks > 1 || !b->one_parent)
+        hipLaunchKernelGGL(k_chunk_starts, dim3(blocks_for(n_chunks + 1, 4)), dim3(256), 0, st, b->d_level,
+                           b->nodes_used, n_chunks, b->d_chunks);
     if (b->one_parent)
-        hipLaunchKernelGGL(k_mark_chunks, dim3(n_chunks), dim3(kChunkWG), 0, st, b->d_nodes, b->d_chunks, b->d_level,
-                           b->d_wide);
+        hipLaunchKernelGGL(k_mark_chunks, dim3(n_chunks), dim3(kChunkWG), 0, st, b->d_nodes, b->nodes_used,
+                           b->d_chunks, b->d_level, b->d_wide);
     uint32_t nb_levels = std::min<uint32_t>(nb, 512);
     hipLaunchKernelGGL(k_level_hist, dim3(nb_levels), dim3(256), 0, st, b->nodes_used, depth, b->d_level, hist);
     // big leaves: counted here, listed below; and whether every node fits a
